@@ -49,16 +49,6 @@ DI fv3 fsub(fv3 a, fv3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
 DI float fdot(fv3 a, fv3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 DI fv3 fcross(fv3 a, fv3 b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
 
-DI bool boxHit(const float4 &lo, const float4 &hi, fv3 o, fv3 inv, float tnear, float tfar, float &tentry) {
-    float tx0 = (lo.x - o.x) * inv.x, tx1 = (hi.x - o.x) * inv.x;
-    float ty0 = (lo.y - o.y) * inv.y, ty1 = (hi.y - o.y) * inv.y;
-    float tz0 = (lo.z - o.z) * inv.z, tz1 = (hi.z - o.z) * inv.z;
-    float t0 = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), tnear));
-    float t1 = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), tfar));
-    tentry = t0;
-    return t0 <= t1;
-}
-
 // Closest hit in [tnear, tfar] of the fp32-rounded ray: global face id (or -1), its
 // t, and the box and triangle tests done. Inlined at every call site: as an
 // out-of-line call, the path kernels save their live path state to scratch around
@@ -67,6 +57,13 @@ DI bool boxHit(const float4 &lo, const float4 &hi, fv3 o, fv3 inv, float tnear, 
 // its lanes' inner-node steps together and then tests the leaves they reached
 // together, instead of running both branches in every step that some lane spends at
 // a leaf; nodes are visited in the same order, so hits are the same.
+//
+// An inner-node step is bound by its vector instructions (the child kernel's are busy
+// 61% of the time, about 40% of them here), so it has no branch of its own: the planes a
+// ray enters and leaves by are chosen by its direction's signs (once per ray), the entry
+// that a pop would take is read along with the node, and the far child is written above
+// the top of the stack whether or not it stays there. Benchmark scene, 512^2, 128 spp, double: child
+// kernel 280 -> 263 ms, AD kernel 326 -> 321 ms; VolPathTracer at 64 spp 34.1 -> 31.3 ms.
 struct TraceHit {
     int face;
     float t;
@@ -75,8 +72,14 @@ struct TraceHit {
 
 // Part of the tree can live in LDS after the traversal stack: its first lds_nodes nodes
 // (the builder numbers the top of the tree breadth-first, so these are its top levels)
-// and, when all nodes fit, also the leaf-ordered triangle records, at LDS float4
-// 4 * nnodes. treeLdsBytes gives the bytes; the launch chooses lds_nodes.
+// and, when all nodes fit, also the leaf-ordered triangle records, after the nodes.
+// treeLdsBytes gives the bytes; the launch chooses lds_nodes. A node in LDS is 14 words:
+// per axis the four planes {left lo, right lo, left hi, right hi}, then the two links.
+// A ray reads, per axis, the pair of planes it enters by and the pair it leaves by, at
+// offsets that depend on its direction's sign alone; the stride of 14 words spreads the
+// nodes that the lanes of a wave are at over the LDS banks.
+constexpr int LDS_NODE = 14;
+HDI size_t ldsNodesBytes(int lds_nodes) { return ((size_t)lds_nodes * LDS_NODE * 4 + 15) / 16 * 16; }
 // Only kernels built with treePrefixInLds<N>() read a part of the nodes from LDS: their
 // traversal tests each node's index against lds_nodes, which the others save by
 // reading LDS only when the whole tree is there (lds_tris), a launch-uniform test.
@@ -85,18 +88,41 @@ struct TraceHit {
 // scene at N = 8 in 7.02 s without and 6.84 s with a prefix of its tree in LDS.
 template <int N> constexpr bool treePrefixInLds() { return N >= 8; }
 HDI size_t treeLdsBytes(const DScene &S, int lds_nodes, bool lds_tris) {
-    return (size_t)lds_nodes * 64 + (lds_tris ? (size_t)S.ntris * 48 : 0);
+    return ldsNodesBytes(lds_nodes) + (lds_tris ? (size_t)S.ntris * 48 : 0);
 }
 // The tree's LDS copy starts after stack_depth stack entries per thread.
-DI const float4 *ldsTree(int stack_depth) { return reinterpret_cast<const float4 *>(s_bvh_stack + stack_depth * blockDim.x); }
+DI float *ldsTree(int stack_depth) { return reinterpret_cast<float *>(s_bvh_stack + stack_depth * blockDim.x); }
 // Copies that part into LDS; called by every thread of the block, at the top of a
 // kernel launched with treeLdsBytes more bytes of dynamic LDS.
 DI void treeToLds(const DScene &S, int lds_nodes, bool lds_tris) {
-    float4 *dst = reinterpret_cast<float4 *>(s_bvh_stack + S.stack_depth * blockDim.x);
-    const int nn = 4 * lds_nodes, nt = lds_tris ? 3 * S.ntris : 0;
-    for (int i = threadIdx.x; i < nn; i += blockDim.x) dst[i] = S.nodes[i];
-    for (int i = threadIdx.x; i < nt; i += blockDim.x) dst[nn + i] = S.tris[i];
+    float *dst = ldsTree(S.stack_depth);
+    for (int i = threadIdx.x; i < lds_nodes; i += blockDim.x) {
+        const float4 *n = S.nodes + 4 * (size_t)i;
+        const float4 a = n[0], b = n[1], c = n[2], e = n[3];
+        float *w = dst + LDS_NODE * i;
+        w[0] = a.x; w[1] = c.x; w[2] = b.x; w[3] = e.x;
+        w[4] = a.y; w[5] = c.y; w[6] = b.y; w[7] = e.y;
+        w[8] = a.z; w[9] = c.z; w[10] = b.z; w[11] = e.z;
+        w[12] = a.w; w[13] = b.w;
+    }
+    float4 *tri = reinterpret_cast<float4 *>(dst + ldsNodesBytes(lds_nodes) / 4);
+    const int nt = lds_tris ? 3 * S.ntris : 0;
+    for (int i = threadIdx.x; i < nt; i += blockDim.x) tri[i] = S.tris[i];
     __syncthreads();
+}
+
+// The two children's entry distances (at least tnear) and whether the ray (origin o,
+// reciprocal direction inv) meets their boxes in [tnear, tfar]. n*: the planes it enters
+// by, f*: those it leaves by, each {left, right}. Choosing them by the direction's sign
+// replaces a minimum and a maximum per plane pair; the distances are the same.
+struct Hit2 { bool l, r; };
+DI Hit2 boxesHit(fv3 o, fv3 inv, float2 nx, float2 ny, float2 nz, float2 fx, float2 fy, float2 fz, float tnear, float tfar,
+                 float &tl, float &tr) {
+    tl = fmaxf(fmaxf((nx.x - o.x) * inv.x, (ny.x - o.y) * inv.y), fmaxf((nz.x - o.z) * inv.z, tnear));
+    tr = fmaxf(fmaxf((nx.y - o.x) * inv.x, (ny.y - o.y) * inv.y), fmaxf((nz.y - o.z) * inv.z, tnear));
+    const float ul = fminf(fminf((fx.x - o.x) * inv.x, (fy.x - o.y) * inv.y), fminf((fz.x - o.z) * inv.z, tfar));
+    const float ur = fminf(fminf((fx.y - o.x) * inv.x, (fy.y - o.y) * inv.y), fminf((fz.y - o.z) * inv.z, tfar));
+    return {tl <= ul, tr <= ur};
 }
 
 template <bool PREFIX = false>
@@ -106,44 +132,51 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
     const float tnear = (float)tnear_, tfar = (float)tfar_;
     TraceHit res{-1, tfar, 0u, 0u};
     if (nnodes == 0) return res;
-    int *stk = s_bvh_stack + threadIdx.x;
     const unsigned stride = blockDim.x;
     const float BEPS = 1e-6f;
     const fv3 inv{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
+    const bool ngx = inv.x < 0.f, ngy = inv.y < 0.f, ngz = inv.z < 0.f;   // entered by the high planes
     float best = tfar;
+    const float *lds = ldsTree(stack_depth);
+    const float *lx = lds + (ngx ? 2 : 0), *ly = lds + (ngy ? 6 : 4), *lz = lds + (ngz ? 10 : 8);
+    const float *gx = lds + (ngx ? 0 : 2), *gy = lds + (ngy ? 4 : 6), *gz = lds + (ngz ? 8 : 10);
     int face = -1;
-    int sp = 0;
     int node = 0;
     uint32_t nbox = 0, ntri = 0;
     constexpr int DONE = INT_MIN;   // no leaf encodes to it: leaves hold >= 1 triangle of < 2^27
+    int *top = s_bvh_stack + threadIdx.x;   // the top stack entry; the bottom one is DONE
+    *top = DONE;
     while (node != DONE) {
         // inner nodes until this lane reaches a leaf or runs out of nodes; the wave then
         // tests the leaves it reached together
         while (node >= 0) {
-            float4 a, b, c, e;
+            const int popped = *top;   // read with the node, so that a pop waits for nothing more
+            float2 nx, ny, nz, fx, fy, fz;
+            int cl, cr;
             if (PREFIX ? node < lds_nodes : lds_tris) {
-                const float4 *n = ldsTree(stack_depth) + 4 * node;
-                a = n[0]; b = n[1]; c = n[2]; e = n[3];
+                const int w = LDS_NODE * node;
+                auto pair = [w](const float *p) { return *reinterpret_cast<const float2 *>(p + w); };
+                nx = pair(lx); ny = pair(ly); nz = pair(lz);
+                fx = pair(gx); fy = pair(gy); fz = pair(gz);
+                const float2 links = pair(lds + 12);
+                cl = __float_as_int(links.x); cr = __float_as_int(links.y);
             } else {
                 const float4 *n = nodes + 4 * (size_t)node;
-                a = n[0]; b = n[1]; c = n[2]; e = n[3];
+                const float4 a = n[0], b = n[1], c = n[2], e = n[3];
+                nx = ngx ? float2{b.x, e.x} : float2{a.x, c.x}; fx = ngx ? float2{a.x, c.x} : float2{b.x, e.x};
+                ny = ngy ? float2{b.y, e.y} : float2{a.y, c.y}; fy = ngy ? float2{a.y, c.y} : float2{b.y, e.y};
+                nz = ngz ? float2{b.z, e.z} : float2{a.z, c.z}; fz = ngz ? float2{a.z, c.z} : float2{b.z, e.z};
+                cl = __float_as_int(a.w); cr = __float_as_int(b.w);
             }
             float tl, tr;
             nbox += 2;
-            bool hl = boxHit(a, b, o, inv, tnear, best, tl);
-            bool hr = boxHit(c, e, o, inv, tnear, best, tr);
-            int cl = __float_as_int(a.w), cr = __float_as_int(b.w);
-            if (hl && hr) {
-                if (tr < tl) { int t = cl; cl = cr; cr = t; }
-                stk[stride * sp++] = cr;
-                node = cl;
-            } else if (hl) {
-                node = cl;
-            } else if (hr) {
-                node = cr;
-            } else {
-                node = sp == 0 ? DONE : stk[stride * --sp];
-            }
+            const Hit2 hit = boxesHit(o, inv, nx, ny, nz, fx, fy, fz, tnear, best, tl, tr);
+            const bool hl = hit.l, hr = hit.r;
+            const bool right = hr && (!hl || tr < tl);   // the right child is the next node
+            top[stride] = right ? cl : cr;   // the other one; above the top unless both are hit
+            node = right ? cr : cl;
+            if (!(hl || hr)) node = popped;
+            top = hl && hr ? top + stride : hl || hr ? top : top - stride;
         }
         if (node == DONE) break;
         int enc = ~node;
@@ -152,7 +185,7 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
         for (int k = first; k < first + cnt; ++k) {
             float4 v0, e1, e2;
             if (lds_tris) {
-                const float4 *tp = ldsTree(stack_depth) + 4 * nnodes + 3 * k;
+                const float4 *tp = reinterpret_cast<const float4 *>(lds + ldsNodesBytes(nnodes) / 4) + 3 * k;
                 v0 = tp[0]; e1 = tp[1]; e2 = tp[2];
             } else {
                 const float4 *tp = tris + 3 * (size_t)k;
@@ -172,7 +205,8 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
             float t = fdot(E2, q) * idet;
             if (t >= tnear && t <= best) { best = t; face = __float_as_int(v0.w); }
         }
-        node = sp == 0 ? DONE : stk[stride * --sp];
+        node = *top;
+        top -= stride;
     }
     res.face = face;
     res.t = best;

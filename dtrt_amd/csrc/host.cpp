@@ -1008,8 +1008,9 @@ bool Scene::build() {
     if (!buildBvh(tri, fshape, bvh)) return false;
     S.nnodes = (int)(bvh.nodes.size() / 4);
     S.ntris = (int)tri.size();
-    // a lane's stack holds at most one entry per inner node on its path (depth - 1)
-    S.stack_depth = std::min(DTRT_BVH_STACK, std::max(1, bvh.depth));
+    // a lane's stack holds its end mark and at most one entry per inner node on its path
+    // (depth - 1; the wrapper of a single leaf counts as one)
+    S.stack_depth = std::min(DTRT_BVH_STACK, std::max(2, bvh.depth));
     S.nodes = upload(bvh.nodes);
     S.tris = upload(bvh.tris);
     S.V = upload(V); S.Vd = upload(Vd); S.Nrm = upload(Nrm); S.Nd = upload(Nd);

@@ -1513,7 +1513,7 @@ template <class K> static size_t treeLdsFor(K kern, unsigned blk, const DScene &
         Pl.lds_nodes = S.nnodes;
         Pl.lds_tris = 1;
     } else if (prefix) {
-        Pl.lds_nodes = (int)std::min<size_t>((size_t)S.nnodes, spare / 64);
+        Pl.lds_nodes = (int)std::min<size_t>((size_t)S.nnodes, spare / (LDS_NODE * 4 + 1));
         if (Pl.lds_nodes < 64) Pl.lds_nodes = 0;
     }
     const size_t tb = treeLdsBytes(S, Pl.lds_nodes, Pl.lds_tris != 0);
