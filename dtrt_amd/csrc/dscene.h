@@ -96,6 +96,7 @@ DI float *ldsTree(int stack_depth) { return reinterpret_cast<float *>(s_bvh_stac
 // kernel launched with treeLdsBytes more bytes of dynamic LDS.
 DI void treeToLds(const DScene &S, int lds_nodes, bool lds_tris) {
     float *dst = ldsTree(S.stack_depth);
+#pragma unroll 2
     for (int i = threadIdx.x; i < lds_nodes; i += blockDim.x) {
         const float4 *n = S.nodes + 4 * (size_t)i;
         const float4 a = n[0], b = n[1], c = n[2], e = n[3];
@@ -107,6 +108,7 @@ DI void treeToLds(const DScene &S, int lds_nodes, bool lds_tris) {
     }
     float4 *tri = reinterpret_cast<float4 *>(dst + ldsNodesBytes(lds_nodes) / 4);
     const int nt = lds_tris ? 3 * S.ntris : 0;
+#pragma unroll 4
     for (int i = threadIdx.x; i < nt; i += blockDim.x) tri[i] = S.tris[i];
     __syncthreads();
 }

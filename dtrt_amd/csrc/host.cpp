@@ -666,6 +666,11 @@ struct Bump {
 // The scratch-only render's child queue must hold at least this much; below it the
 // render is refused (the exact overflow replay would still finish, in many rounds).
 constexpr uint64_t NOALLOC_MIN_QUEUE = uint64_t(16) << 20;
+// AD samples in flight at once (the slots of the staged AD kernels' path state).
+#ifndef AD_SLOTS_LOG
+#define AD_SLOTS_LOG 22
+#endif
+constexpr uint64_t AD_SLOTS = uint64_t(1) << AD_SLOTS_LOG;
 
 struct Scene : Obj {
     Scene() : Obj(T_SCENE) {}
@@ -677,7 +682,7 @@ struct Scene : Obj {
         for (void *p : pe_bufs) (void)hipFree(p);
         for (auto *b : {&edgebuf, &ecdfbuf, &lightbuf, &refitbuf, &shapecdfbuf}) if (b->p) (void)hipFree(b->p);
         for (auto &b : bufs) if (b.p) (void)hipFree(b.p);
-        for (auto *b : {&acc, &acc_pe, &queue, &qcount, &stats, &work, &outbuf, &ovf[0], &ovf[1], &viewbuf, &tunebuf})
+        for (auto *b : {&acc, &acc_pe, &queue, &qcount, &stats, &work, &outbuf, &ovf[0], &ovf[1], &viewbuf, &tunebuf, &adstate})
             if (b->p) (void)hipFree(b->p);
         for (auto &e : ev) if (e) (void)hipEventDestroy(e);
         if (caller_ev) (void)hipEventDestroy(caller_ev);
@@ -692,7 +697,7 @@ struct Scene : Obj {
     std::vector<Medium *> media;
     DScene S;
     std::vector<DevBuf> bufs;
-    DevBuf acc, acc_pe, queue, qcount, stats, work, outbuf, ovf[2], viewbuf;
+    DevBuf acc, acc_pe, queue, qcount, stats, work, outbuf, ovf[2], viewbuf, adstate;
     std::vector<DMedium> hmed;   // host copy of the device media records
     struct PECache { int npe = 0; double pe_sum = 0; const double *cdf = nullptr; const float *pe = nullptr; };
     std::vector<void *> pe_bufs;   // device buffers of the primary-edge cache (freed when geometry changes)
@@ -747,6 +752,18 @@ struct Scene : Obj {
     // 262 -> 220 ms in float, against 64.
     int tune_ad_block = 64, tune_child_block = 256;
     DevBuf tunebuf;
+    unsigned ad_slots = 0;   // samples that adstate holds
+    // The path state of the staged AD kernels for chunks of up to `chunk` samples.
+    bool useAdState(RenderParams &P, uint64_t chunk) {
+        const unsigned want = (unsigned)std::min<uint64_t>(AD_SLOTS, (chunk + 63) / 64 * 64);
+        if (ad_slots < want) {
+            if (!ensure(adstate, adStateBytes(nder, S.f64 != 0, want))) return false;
+            ad_slots = want;
+        }
+        P.ad_state = static_cast<char *>(adstate.p);
+        P.ad_slots = ad_slots;
+        return true;
+    }
 
     template <class T> const T *upload(const std::vector<T> &v) {
         if (v.empty()) return nullptr;
@@ -790,7 +807,7 @@ struct Scene : Obj {
     bool captureViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, float *const *images);
     int replayViews(const uint64_t *seeds);
     std::vector<void *> graphBuffers() const {
-        return {viewbuf.p, acc.p, acc_pe.p, queue.p, qcount.p, stats.p, work.p, ovf[0].p, ovf[1].p};
+        return {viewbuf.p, acc.p, acc_pe.p, queue.p, qcount.p, stats.p, work.p, ovf[0].p, ovf[1].p, adstate.p};
     }
     bool setupViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, std::vector<DView> &hv,
                     std::vector<uint64_t> &pe_total, Bump *pool = nullptr);
@@ -1361,7 +1378,7 @@ bool Scene::setupViews(int nv, const Camera *const *cams, const dtrt_render_opti
     return true;
 }
 
-constexpr uint64_t FIRST_CHUNK = uint64_t(1) << 16;  // before the children-per-sample rate is known
+constexpr uint64_t FIRST_CHUNK = uint64_t(1) << 18;  // before the children-per-sample rate is known
 
 // All views in one pass: their AD samples form one global sample space (launched in
 // the same chunks), their primary-edge samples follow view by view, and each view's
@@ -1425,11 +1442,16 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
                         std::to_string(DTRT_SCRATCH_BYTES >> 20) + " MiB scratch area holds (accumulators " +
                         std::to_string((img + (size_t)nder * npix * 3) * es >> 20) + " MiB, plus a queue of at least " +
                         std::to_string(NOALLOC_MIN_QUEUE >> 20) + " MiB)");
-        Q = static_cast<char *>(pool->take(qbytes));
-        cap = std::min<uint64_t>(qbytes / P.rec_stride, 0xFFFFFFF0ull);
+        // a quarter of it for the path state, as many samples in flight as fit
+        P.ad_slots = (unsigned)std::min<uint64_t>(AD_SLOTS, (qbytes / 4 - adStateBytes(nder, S.f64 != 0, 0)) / adSlotBytes(nder, S.f64 != 0) / 64 * 64);
+        P.ad_state = static_cast<char *>(pool->take(adStateBytes(nder, S.f64 != 0, P.ad_slots)));
+        const uint64_t qleft = pool->left / 256 * 256;
+        Q = static_cast<char *>(pool->take(qleft));
+        cap = std::min<uint64_t>(qleft / P.rec_stride, 0xFFFFFFF0ull);
     } else {
         cap = std::max<uint64_t>(128, std::min<uint64_t>(queue_budget / P.rec_stride, 0xFFFFFFF0ull));
         max_chunk = std::min<uint64_t>(tune_max_chunk, std::max<uint64_t>(total, 64));
+        if (ad_kind == AD_VOLPATH && !useAdState(P, max_chunk)) return false;
         if (!ensure(acc, img * es) || !ensure(acc_pe, (size_t)nder * npix * 3 * es) || !ensure(qcount, 64) ||
             !ensure(stats, 64 * 4) || !ensure(work, 16 * 8) || !ensure(queue, (size_t)cap * P.rec_stride) ||
             !ensure(ovf[0], (size_t)max_chunk * 16) || !ensure(ovf[1], (size_t)max_chunk * 16))
@@ -1589,6 +1611,8 @@ bool Scene::captureViews(int nv, const Camera *const *cams, const dtrt_render_op
     const uint64_t cap = std::max<uint64_t>(128, std::min<uint64_t>(queue_budget / P.rec_stride, 0xFFFFFFF0ull));
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
+    P.ad_state = static_cast<char *>(adstate.p);
+    P.ad_slots = ad_slots;
     int dev = 0, ncu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1779,6 +1803,8 @@ bool Scene::captureStep(StepArgs &a) {
     const uint64_t cap = std::max<uint64_t>(128, std::min<uint64_t>(queue_budget / P.rec_stride, 0xFFFFFFF0ull));
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
+    P.ad_state = static_cast<char *>(adstate.p);
+    P.ad_slots = ad_slots;
     int dev = 0, ncu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));

@@ -1,11 +1,12 @@
 // gfx950 kernels of the forward-mode AD volumetric path tracer.
 //
-//  k_ad_paths<N>    one thread per AD path sample (pixel x spp). Runs the dual-number
-//                   estimator LiAD (volpathAD.cpp:145-620) iteratively, accumulates the
-//                   interior terms, and pushes every primal sub-path the boundary terms
-//                   need (2 per accepted edge sample, 1 per Lins sample) into an HBM queue.
-//  k_ad_refill<N>   the same for N >= 8 (one wave per SIMD), with per-bounce lane refill:
-//                   a lane whose path has ended starts the wave's next sample.
+//  k_ad_bounce<N>, k_ad_edges<N>, k_ad_finish<N> (ad_stages.h)
+//                   the AD path samples (pixel x spp) of VolPathTracerAD: the dual-number
+//                   estimator LiAD (volpathAD.cpp:145-620) one bounce per launch over the
+//                   paths still alive. They sum the interior terms and push every primal
+//                   sub-path the boundary terms need (2 per accepted edge sample, 1 per
+//                   Lins sample) into an HBM queue.
+//  k_ad_paths<N>    the same for the surface-only integrators, one thread per sample.
 //  k_children<N>    one thread per queued sub-path: primal Li / Lins estimate, scattered
 //                   with its per-lane weights into the derivative accumulators.
 //  k_primary<N>     primary-edge samples (integratorAD.cpp:100-165): 2 camera sub-paths each.
@@ -57,27 +58,21 @@ HDI unsigned blockOr64(int b) { return b == 128 || b == 256 ? (unsigned)b : 64u;
 #define CHILD_WAVES_F64 2   // heterogeneous-medium scene, 512^2, 128 spp, nder 3, child kernel per render: 2 waves 413 ms, 4 waves 464 ms (1 wave: 1.5x 2)
 #endif
 #ifndef AD_WAVES_PER_SIMD
-#define AD_WAVES_PER_SIMD (kF64 ? AD_WAVES_F64 : 2)
+#define AD_WAVES_PER_SIMD (kF64 ? 1 : 2)   // the surface-only AD kernel and the adjoint
 #endif
-#ifndef AD_WAVES_F64
-#define AD_WAVES_F64 1      // 1 wave: 394 ms, 2 waves: 514 ms per render's AD kernel (same scene and size)
+template <int N> constexpr int adWaves() { return N >= 8 ? 1 : AD_WAVES_PER_SIMD; }
+// The staged AD kernels (ad_stages.h): work-groups of four waves, one per SIMD, which share
+// one copy of the tree. Waves per SIMD that the register allocator leaves room for: in
+// double one, since their spills at two cost more than a second wave gives (benchmark scene,
+// 512^2, 128 spp, nder 3, AD time per render: bounces at one wave 183 ms, at two 251; edge
+// terms at one wave 174, at two 184, at three 209); in float two (333x250, 48 spp: bounces at
+// two 20.3 ms, at one 22.0; edge terms the same at two, three and four).
+constexpr int AD_STAGE_BLOCK = 256;
+#ifndef AD_BOUNCE_WAVES
+#define AD_BOUNCE_WAVES (kF64 ? 1 : 2)
 #endif
-// Dual widths from which the VolPathTracerAD samples run in k_ad_refill (per-bounce
-// lane refill) at one wave per SIMD, with the whole 512-entry register file, rather
-// than spilling kilobytes per lane to scratch.
-#ifndef AD_REFILL_MIN_N
-#define AD_REFILL_MIN_N (kF64 ? AD_REFILL_MIN_N_F64 : 8)
-#endif
-#ifndef AD_REFILL_MIN_N_F64
-#define AD_REFILL_MIN_N_F64 8
-#endif
-template <int N> constexpr bool adRefill() { return N >= AD_REFILL_MIN_N; }
-template <int N> constexpr int adWaves() { return adRefill<N>() ? 1 : AD_WAVES_PER_SIMD; }
-// Grid of k_ad_refill: waves per CU sharing a launch's samples (measured on the
-// 100K-face dielectric scene at nder 8: in float 64 beats 32 and 128; in double the
-// AD kernel takes 8.16, 7.76, 7.62, 7.48, 7.84, 8.78 s at 4, 8, 16, 32, 64, 128).
-#ifndef AD_REFILL_WAVES_PER_CU
-#define AD_REFILL_WAVES_PER_CU (kF64 ? 32 : 64)
+#ifndef AD_EDGE_WAVES
+#define AD_EDGE_WAVES (kF64 ? 1 : 2)
 #endif
 
 DI uint32_t xcdRemap(uint32_t b, uint32_t nb) {
@@ -520,7 +515,7 @@ DI void adPathSample(Tracer<N> &T, const RenderParams &P, const DView &vw, Rng &
 // Normal pass: samples s0 .. s0+nsamp-1. Replay pass (replay != nullptr): entries
 // {sid lo, sid hi, children delivered, 0} of samples whose pushes overflowed.
 // Samples that overflow (again) are appended to ovf.
-template <int N, int I>   // I: AdKind
+template <int N, int I>   // I: AD_PATH or AD_DIRECT
 __global__ __launch_bounds__(MAX_BLOCK, adWaves<N>()) void k_ad_paths(DScene S, RenderParams P, uint64_t s0, uint64_t nsamp,
                                                     const uint4 *replay, real *acc, char *q, unsigned *qcount,
                                                     unsigned *stats, uint4 *ovf, unsigned *ovf_count,
@@ -546,8 +541,7 @@ __global__ __launch_bounds__(MAX_BLOCK, adWaves<N>()) void k_ad_paths(DScene S, 
     Rng r;
     r.init(vw.seed, ls);
     if (active) {
-        if constexpr (I == AD_VOLPATH) adPathSample<N, AdjPass::NONE>(T, P, vw, r, pixel, L, u, stats, nullptr);
-        else adSurfaceSample<N, I == AD_DIRECT>(T, P, vw, r, pixel, L, u, stats);
+        adSurfaceSample<N, I == AD_DIRECT>(T, P, vw, r, pixel, L, u, stats);
     }
     const bool done = u.failed_at == Pusher::NO_FAIL;
     if (active && !done) ovf[atomicAdd(ovf_count, 1u)] = make_uint4((uint32_t)sid, (uint32_t)(sid >> 32), u.failed_at, 0u);
@@ -610,10 +604,11 @@ DI bool adBegin(const RenderParams &P, const DView &vw, Rng &r, int pixel, AdSta
     return st.mode != 0;
 }
 
-// One iteration of adPathSample's bounce loop (forward pass). False when the path ends.
-template <int N>
-DI bool adBounce(Tracer<N> &T, const RenderParams &P, Rng &r, int pixel, AdState<N> &st, Ds<N> &L, Pusher &u,
-                 unsigned *stats) {
+// One iteration of adPathSample's bounce loop (forward pass), its edge term left in eo.
+// False when the path ends.
+template <int N, class EdgeOut>
+DI bool adBounce(Tracer<N> &T, const RenderParams &P, Rng &r, AdState<N> &st, Ds<N> &L, Pusher &u, unsigned *stats,
+                 EdgeOut &eo) {
     constexpr AdjPass A = AdjPass::NONE;
     const AdjCtx *ac = nullptr;
     const DScene &S = T.S;
@@ -635,93 +630,16 @@ DI bool adBounce(Tracer<N> &T, const RenderParams &P, Rng &r, int pixel, AdState
 #define AD_BOUNCE_END return false
 #define AD_WALK_DEFERRED(kind, surf, add, cp) \
     { st.walk = (kind); st.walk_surf = (surf); st.walk_add = (add); st.walk_cpdf = (cp); }
+#define AD_EDGE_DEFERRED(vol, x, hit, rdin, thrv, betav, med, depth) \
+    { if (S.edges_valid) eo.put(vol, x, hit, rdin, thrv, betav, med, depth); }
 #include "ad_bounce.inc"
+#undef AD_EDGE_DEFERRED
 #undef AD_WALK_DEFERRED
 #undef AD_BOUNCE_END
     return mode != 0;
 }
 
-// VolPathTracerAD samples with per-bounce lane refill (same estimator and random
-// streams as k_ad_paths<N, AD_VOLPATH>), for the dual widths that run one wave per
-// SIMD: there the hardware has few other waves to switch to, and the lanes of a wave
-// that wait for its longest path dominate. Each wave owns the contiguous range of
-// `per_wave` sample indices of its block; a lane whose path has ended takes the
-// wave's next sample before the next bounce, until the range is used up. Finished
-// samples are summed over the wave per pixel (one atomic per pixel and channel), or
-// listed in ovf when a push overflowed the queue. Indices are into replay[] in a
-// replay pass.
-template <int N>
-__global__ __launch_bounds__(BLOCK, adWaves<N>()) void k_ad_refill(DScene S, RenderParams P, uint64_t s0, uint64_t nsamp,
-                                                     uint64_t per_wave, const uint4 *replay, real *acc, char *q,
-                                                     unsigned *qcount, unsigned *stats, uint4 *ovf, unsigned *ovf_count,
-                                                     unsigned long long *work) {
-    const uint32_t blk = xcdRemap(blockIdx.x, gridDim.x);
-    const uint64_t begin = (uint64_t)blk * per_wave;
-    const uint64_t end = begin < nsamp ? min(nsamp, begin + per_wave) : begin;
-    Tracer<N> T(S);
-    T.useLdsTree(P);
-    AdState<N> st;
-    Ds<N> L;
-    Rng r;
-    Pusher u{q, qcount, 0, 0, 0, 0, 0, Pusher::NO_FAIL};
-    uint64_t sid = 0, next = begin;
-    int pixel = 0;
-    uint32_t nlk = 0;
-    bool alive = false, have = false, exhausted = false;
-    const int nd = P.npix;
-    while (true) {
-        const bool fin = have && !alive;   // the lane's path has ended: add its sample
-        const bool put = fin && u.failed_at == Pusher::NO_FAIL;
-        if (fin && !put) ovf[atomicAdd(ovf_count, 1u)] = make_uint4((uint32_t)sid, (uint32_t)(sid >> 32), u.failed_at, 0u);
-        uint64_t pm = __ballot(put);
-        while (pm) {   // wave-uniform: one pixel per round
-            const int lead = __ffsll((unsigned long long)pm) - 1;
-            const int gp0 = __shfl(u.gpix, lead);
-            const bool mine = put && u.gpix == gp0;
-            pm &= ~__ballot(mine);
-#pragma unroll
-            for (int k = 0; k < 3 * (N + 1); ++k) {
-                const int c = k % 3, j = k / 3;
-                real x = mine ? (j == 0 ? L.c[c].v : L.c[c].d[j - 1]) : 0._r;
-                for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-                if ((int)(threadIdx.x & 63) == lead && x != 0._r) unsafeAtomicAdd(acc + ((size_t)j * nd + gp0) * 3 + c, x);
-            }
-        }
-        if (fin) {
-            nlk += r.nlk;
-            have = false;
-        }
-        const bool want = !alive && !exhausted;
-        const uint64_t m = __ballot(want);
-        if (m == 0 && !__any(alive)) break;   // the wave's range is used up
-        if (want) {
-            const uint64_t li = next + __popcll(m & __lanemask_lt());
-            if (li < end) {
-                uint32_t skip = 0;
-                sid = s0 + li;
-                if (replay) {
-                    const uint4 e = replay[li];
-                    sid = (uint64_t)e.x | ((uint64_t)e.y << 32);
-                    skip = e.z;
-                }
-                const int v = viewOf(S, sid);
-                const DView &vw = S.views[v];
-                const uint64_t ls = sid - vw.s0;   // sample index within the view: keys its random stream
-                pixel = (int)(ls / (uint64_t)vw.spp);
-                u = Pusher{q, qcount, vw.pix0 + pixel, v, (ls + 1) << 20, 0, skip, Pusher::NO_FAIL};
-                r.init(vw.seed, ls);
-                L = Ds<N>();
-                have = true;
-                alive = adBegin<N>(P, vw, r, pixel, st);
-            } else {
-                exhausted = true;
-            }
-        }
-        next += (uint64_t)__popcll(m);
-        if (alive) alive = adBounce<N>(T, P, r, pixel, st, L, u, stats);
-    }
-    flushWork(work, 0, T.nbox, T.ntri, nlk, T.nseg);
-}
+#include "ad_stages.h"
 
 // The primal integrators: one thread per sample s0 .. s0+n-1 of view 0 (sample k of
 // pixel p is p*spp + k), a jittered camera ray and the estimator of KIND:
@@ -1449,6 +1367,9 @@ template <int N> struct WidthOps {
     static void launchAd(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const uint4 *replay, real *acc,
                          char *q, unsigned *qc, unsigned *st, uint4 *ovf, unsigned *ovf_count, unsigned long long *wk,
                          hipStream_t sm);
+    static void launchAdStages(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const uint4 *replay,
+                               real *acc, char *q, unsigned *qc, unsigned *st, uint4 *ovf, unsigned *ovf_count,
+                               unsigned long long *wk, hipStream_t sm);
     static void launchChildren(const DScene &S, const RenderParams &P, const char *q, unsigned *qc, real *acc,
                                real *acc_pe, unsigned long long *wk, unsigned grid, hipStream_t sm);
     static void launchPrimary(const DScene &S, const RenderParams &P, int view, uint64_t s0, uint64_t n, uint64_t total,
@@ -1552,22 +1473,53 @@ template <int N> void WidthOps<N>::launchAd(const DScene &S, const RenderParams 
         const size_t tl = treeLdsFor(k_ad_paths<N, AD_DIRECT>, blk, S, Pl, treePrefixInLds<N>());
         hipLaunchKernelGGL((k_ad_paths<N, AD_DIRECT>), dim3(nb), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, s0, n, replay,
                            acc, q, qc, st, ovf, ovf_count, wk);
-    } else if constexpr (adRefill<N>()) {
-        // one wave per block, AD_REFILL_WAVES_PER_CU of them per CU share the samples
-        int dev = 0, ncu = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        const uint64_t waves = (uint64_t)std::max(ncu, 1) * AD_REFILL_WAVES_PER_CU;
-        const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>((n + BLOCK - 1) / BLOCK, waves));
-        const uint64_t per_wave = (n + grid - 1) / grid;
-        const size_t tl = treeLdsFor(k_ad_refill<N>, BLOCK, S, Pl, treePrefixInLds<N>());
-        // one wave per block: each owns a contiguous range of samples
-        hipLaunchKernelGGL(k_ad_refill<N>, dim3((unsigned)grid), dim3(BLOCK), traceLds(BLOCK, S.stack_depth) + tl, sm, S, Pl, s0, n,
-                           per_wave, replay, acc, q, qc, st, ovf, ovf_count, wk);
     } else {
-        const size_t tl = treeLdsFor(k_ad_paths<N, AD_VOLPATH>, blk, S, Pl, treePrefixInLds<N>());
-        hipLaunchKernelGGL((k_ad_paths<N, AD_VOLPATH>), dim3(nb), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, s0, n, replay,
-                           acc, q, qc, st, ovf, ovf_count, wk);
+        launchAdStages(S, P, s0, n, replay, acc, q, qc, st, ovf, ovf_count, wk, sm);
+    }
+}
+// Blocks of `blk` threads and `lds` bytes of kernel `fn` that the device holds at once.
+template <class K> static unsigned residentBlocks(K fn, unsigned blk, size_t lds) {
+    int dev = 0, ncu = 0, per = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, (int)blk, lds) != hipSuccess || per <= 0) {
+        (void)hipGetLastError();
+        per = 1;
+    }
+    return (unsigned)std::max(ncu, 1) * (unsigned)per;
+}
+// A VolPathTracerAD chunk as batches of at most P.ad_slots samples: per bounce one launch
+// of k_ad_bounce and one of k_ad_edges over the paths that are still alive.
+template <int N> void WidthOps<N>::launchAdStages(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n,
+                                                  const uint4 *replay, real *acc, char *q, unsigned *qc, unsigned *st,
+                                                  uint4 *ovf, unsigned *ovf_count, unsigned long long *wk, hipStream_t sm) {
+    const unsigned blk = AD_STAGE_BLOCK, wpb = blk / 64;
+    RenderParams Pb = P, Pe = P;
+    const size_t lb = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_bounce<N>, blk, S, Pb, treePrefixInLds<N>());
+    const size_t le = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_edges<N>, blk, S, Pe, treePrefixInLds<N>());
+    const unsigned rb = residentBlocks(k_ad_bounce<N>, blk, lb), re = residentBlocks(k_ad_edges<N>, blk, le);
+    const bool edges = P.sppse > 0 && S.edges_valid && (P.mode & (4 | 32)) != 0;
+    AdBatch B{};
+    B.state = P.ad_state;
+    B.n = P.ad_slots;
+    uint32_t *lists = reinterpret_cast<uint32_t *>(P.ad_state + (size_t)B.n * (AdSlots<N>::REALS * sizeof(real) + AdSlots<N>::WORDS * 4));
+    uint32_t *cnt = lists + 3 * (size_t)B.n;
+    B.edges = lists + 2 * (size_t)B.n;
+    for (uint64_t b0 = 0; b0 < n; b0 += B.n) {
+        B.m = (uint32_t)std::min<uint64_t>(B.n, n - b0);
+        B.s0 = s0 + b0;
+        B.replay = replay ? replay + b0 : nullptr;
+        (void)launch_fill32(cnt, 4 * (P.max_bounces + 3), 0u, sm);
+        const unsigned few = (B.m + 4 * wpb - 1) / (4 * wpb);   // blocks beyond get no item (ListShare)
+        for (int k = 0; k <= P.max_bounces; ++k) {
+            B.in = k == 0 ? nullptr : lists + (size_t)(k & 1) * B.n;
+            B.out = lists + (size_t)((k + 1) & 1) * B.n;
+            B.cnt = cnt + 4 * k;
+            hipLaunchKernelGGL(k_ad_bounce<N>, dim3(std::min(rb, few)), dim3(blk), lb, sm, S, Pb, B, q, qc, st, wk);
+            if (edges && k < P.max_bounces)
+                hipLaunchKernelGGL(k_ad_edges<N>, dim3(std::min(re, few)), dim3(blk), le, sm, S, Pe, B, q, qc, st, wk);
+        }
+        hipLaunchKernelGGL(k_ad_finish<N>, dim3((B.m + 255) / 256, 3 * (N + 1)), dim3(256), 0, sm, P, B, acc, ovf, ovf_count);
     }
 }
 template <int N> void WidthOps<N>::launchChildren(const DScene &S, const RenderParams &P, const char *q, unsigned *qc,
@@ -1618,11 +1570,9 @@ template <int N> hipError_t WidthOps<N>::kernelInfo(KernelInfo *out, int cap, in
         std::snprintf(nm, sizeof(nm), LABEL "<%d>", N);                          \
         e = addKernelInfo(FN, nm, BLK, LDS, out, cap, count);                     \
     }
-    if constexpr (adRefill<N>()) {
-        DT_INFO(k_ad_refill<N>, "k_ad_refill", BLOCK, traceLds(BLOCK))
-    } else {
-        DT_INFO((k_ad_paths<N, AD_VOLPATH>), "k_ad_paths", MAX_BLOCK, traceLds(MAX_BLOCK))
-    }
+    DT_INFO(k_ad_bounce<N>, "k_ad_bounce", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
+    DT_INFO(k_ad_edges<N>, "k_ad_edges", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
+    DT_INFO(k_ad_finish<N>, "k_ad_finish", 256, 0)
     DT_INFO((k_ad_paths<N, AD_PATH>), "k_ad_paths/path", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_ad_paths<N, AD_DIRECT>), "k_ad_paths/direct", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO(k_children<N>, "k_children", MAX_BLOCK, traceLds(MAX_BLOCK))

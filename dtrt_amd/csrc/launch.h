@@ -20,8 +20,21 @@ struct RenderParams {
     unsigned qcap;           // child records the queue can hold
     int ad_block, child_block;   // work-group sizes of the AD-path and child kernels (64, 128, 256; 0 = 64)
     int lds_nodes, lds_tris;     // set per launch: the part of the BVH the kernel copies into LDS (treeToLds)
+    char *ad_state;              // path state of the staged AD kernels (adStateBytes) and the samples it holds at once
+    unsigned ad_slots;
     int tree_in_hbm;             // nonzero: no part of the BVH goes into LDS (a test setting)
 };
+
+// Bytes of the staged AD kernels' path state for `slots` samples in flight: per slot the
+// reals and words of AdSlots (ad_stages.h) and three list entries, then the counters of
+// every bounce.
+constexpr int AD_SLOT_WORDS = 15;
+constexpr int adSlotReals(int nder) { return 12 * (nder + 1) + 16; }
+constexpr int AD_MAX_BOUNCES = 200;
+constexpr uint64_t adSlotBytes(int nder, bool f64) { return (uint64_t)adSlotReals(nder) * (f64 ? 8 : 4) + AD_SLOT_WORDS * 4 + 12; }
+constexpr uint64_t adStateBytes(int nder, bool f64, uint64_t slots) {
+    return slots * adSlotBytes(nder, f64) + 16 * (AD_MAX_BOUNCES + 3);
+}
 
 // Counters written by the kernels (warnings the reference prints, as counts).
 enum Stat {
