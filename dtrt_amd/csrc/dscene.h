@@ -297,21 +297,51 @@ DI bool isTransition(const DShape &sh) { return sh.med_ext >= 0 || sh.med_int >=
 DI const DBsdf &bsdfOf(const DScene &S, const DShape &sh) { return S.bsdfs[sh.bsdf_id]; }
 
 // -------------------------------------------------------------- media
-// gridvolume.h:144-201 — node-centred trilinear lookup, zero outside [0, res-2] cells
-DI real trilinear(const float *data, const int *res, f3 g, int ch, int nch) {
+// Cell of a node-centred grid coordinate, and its eight corner values (channel ch of nch).
+struct GridCell {
+    int x, y, z;
+    real fx, fy, fz;
+};
+DI bool gridCell(const int *res, f3 g, GridCell &c) {
     real fx0 = floor(g.x), fy0 = floor(g.y), fz0 = floor(g.z);
     // bounds are tested on the floats first so NaN / huge coordinates never reach the int conversion
     if (!(fx0 >= 0._r && fy0 >= 0._r && fz0 >= 0._r && fx0 < (real)(res[0] - 1) && fy0 < (real)(res[1] - 1) && fz0 < (real)(res[2] - 1)))
-        return 0._r;
-    int x1 = (int)fx0, y1 = (int)fy0, z1 = (int)fz0;
-    real fx = g.x - fx0, fy = g.y - fy0, fz = g.z - fz0;
-    size_t sy = (size_t)res[0] * nch, sz = sy * res[1];
-    const float *b = data + (size_t)z1 * sz + (size_t)y1 * sy + (size_t)x1 * nch + ch;
-    real d000 = __ldg(b), d001 = __ldg(b + nch), d010 = __ldg(b + sy), d011 = __ldg(b + sy + nch);
-    real d100 = __ldg(b + sz), d101 = __ldg(b + sz + nch), d110 = __ldg(b + sz + sy), d111 = __ldg(b + sz + sy + nch);
-    real _fx = 1._r - fx, _fy = 1._r - fy, _fz = 1._r - fz;
-    return ((d000 * _fx + d001 * fx) * _fy + (d010 * _fx + d011 * fx) * fy) * _fz +
-           ((d100 * _fx + d101 * fx) * _fy + (d110 * _fx + d111 * fx) * fy) * fz;
+        return false;
+    c.x = (int)fx0; c.y = (int)fy0; c.z = (int)fz0;
+    c.fx = g.x - fx0; c.fy = g.y - fy0; c.fz = g.z - fz0;
+    return true;
+}
+struct Corners {
+    real d000, d001, d010, d011, d100, d101, d110, d111;
+};
+// Both x neighbours of a row of a one-channel grid in one 8-byte load (4-byte aligned).
+struct __attribute__((packed, aligned(4))) FloatPair {
+    float a, b;
+};
+DI void loadCorners(const float *data, const int *res, const GridCell &c, Corners &k) {
+    const size_t sy = (size_t)res[0], sz = sy * res[1];
+    const float *p = data + (size_t)c.z * sz + (size_t)c.y * sy + c.x;
+    auto row = [](const float *q) { return *reinterpret_cast<const FloatPair *>(q); };
+    const FloatPair a = row(p), b = row(p + sy), e = row(p + sz), f = row(p + sz + sy);
+    k.d000 = a.a; k.d001 = a.b; k.d010 = b.a; k.d011 = b.b;
+    k.d100 = e.a; k.d101 = e.b; k.d110 = f.a; k.d111 = f.b;
+}
+// gridvolume.h:144-201 — node-centred trilinear lookup, zero outside [0, res-2] cells
+DI real trilinear(const float *data, const int *res, f3 g, int ch, int nch) {
+    GridCell c;
+    if (!gridCell(res, g, c)) return 0._r;
+    Corners k;
+    if (nch == 1) {
+        loadCorners(data, res, c, k);
+    } else {
+        const size_t sy = (size_t)res[0] * nch, sz = sy * res[1];
+        const float *b = data + (size_t)c.z * sz + (size_t)c.y * sy + (size_t)c.x * nch + ch;
+        k.d000 = __ldg(b); k.d001 = __ldg(b + nch); k.d010 = __ldg(b + sy); k.d011 = __ldg(b + sy + nch);
+        k.d100 = __ldg(b + sz); k.d101 = __ldg(b + sz + nch); k.d110 = __ldg(b + sz + sy); k.d111 = __ldg(b + sz + sy + nch);
+    }
+    real _fx = 1._r - c.fx, _fy = 1._r - c.fy, _fz = 1._r - c.fz;
+    return ((k.d000 * _fx + k.d001 * c.fx) * _fy + (k.d010 * _fx + k.d011 * c.fx) * c.fy) * _fz +
+           ((k.d100 * _fx + k.d101 * c.fx) * _fy + (k.d110 * _fx + k.d111 * c.fx) * c.fy) * c.fz;
 }
 template <int N> DI Df<N> trilinearAD(const float *data, const int *res, const Dv<N> &g, int ch, int nch) {
     real fx0 = floor(g.x.v), fy0 = floor(g.y.v), fz0 = floor(g.z.v);
@@ -364,18 +394,11 @@ template <int N> DI Dv<N> toGridAD(const DMedium &m, const Dv<N> &p, bool albedo
     }
     return g;
 }
-// Cell of a node-centred grid coordinate, with the bounds test of trilinear().
-struct GridCell {
-    int x, y, z;
-    real fx, fy, fz;
-};
-DI bool gridCell(const int *res, f3 g, GridCell &c) {
-    real fx0 = floor(g.x), fy0 = floor(g.y), fz0 = floor(g.z);
-    if (!(fx0 >= 0._r && fy0 >= 0._r && fz0 >= 0._r && fx0 < (real)(res[0] - 1) && fy0 < (real)(res[1] - 1) && fz0 < (real)(res[2] - 1)))
-        return false;
-    c.x = (int)fx0; c.y = (int)fy0; c.z = (int)fz0;
-    c.fx = g.x - fx0; c.fy = g.y - fy0; c.fz = g.z - fz0;
-    return true;
+// Gradient in grid coordinates to world space: (w2v, gscale) transposed.
+DI f3 gradToWorld(const DMedium &m, f3 g) {
+    const f3 s{g.x * m.gscale[0], g.y * m.gscale[1], g.z * m.gscale[2]};
+    const float *w = m.w2v;
+    return f3{w[0] * s.x + w[4] * s.y + w[8] * s.z, w[1] * s.x + w[5] * s.y + w[9] * s.z, w[2] * s.x + w[6] * s.y + w[10] * s.z};
 }
 
 template <int N> DI Df<N> lookupDensityAD(const DMedium &m, const Dv<N> &p) {
@@ -453,26 +476,90 @@ DI bool aabbIntersect(const float *lo, const float *hi, f3 o, f3 d, real &nearT,
     return true;
 }
 
-// heterogeneous.cpp:121-141 — derivative of the optical depth along a segment
+// The grid coordinate along a ray, which is affine in t. In double it is taken from the
+// coordinate of the origin and of the direction (one FMA per axis and lookup); the float
+// kernels transform each point, so that their free-flight decisions keep their rounding.
+struct GridRay {
+    f3 o, d;
+    DI GridRay(const DMedium &m, f3 ro, f3 rd) {
+        if constexpr (kF64) {
+            o = toGrid(m, ro);
+            const f3 v = xform33(m.w2v, rd);
+            d = f3{v.x * m.gscale[0], v.y * m.gscale[1], v.z * m.gscale[2]};
+        } else {
+            o = ro;
+            d = rd;
+        }
+    }
+    DI f3 at(const DMedium &m, real t) const {
+        if constexpr (kF64) return f3{o.x + d.x * t, o.y + d.y * t, o.z + d.z * t};
+        else return toGrid(m, o + d * t);
+    }
+};
+// Trilinear density at grid coordinate g and its gradient there (zero outside the grid).
+DI real densityGrad(const DMedium &m, f3 g, f3 &grad) {
+    grad = f3{0, 0, 0};
+    GridCell c;
+    if (!gridCell(m.res, g, c)) return 0._r;
+    Corners k;
+    loadCorners(m.density, m.res, c, k);
+    const real vx0 = k.d000 + (k.d001 - k.d000) * c.fx, vx1 = k.d010 + (k.d011 - k.d010) * c.fx;
+    const real vx2 = k.d100 + (k.d101 - k.d100) * c.fx, vx3 = k.d110 + (k.d111 - k.d110) * c.fx;
+    const real vy0 = vx0 + (vx1 - vx0) * c.fy, vy1 = vx2 + (vx3 - vx2) * c.fy;
+    const real _fy = 1._r - c.fy, _fz = 1._r - c.fz;
+    grad.x = ((k.d001 - k.d000) * _fy + (k.d011 - k.d010) * c.fy) * _fz + ((k.d101 - k.d100) * _fy + (k.d111 - k.d110) * c.fy) * c.fz;
+    grad.y = (vx1 - vx0) * _fz + (vx3 - vx2) * c.fz;
+    grad.z = vy1 - vy0;
+    return vy0 + (vy1 - vy0) * c.fz;
+}
+// w * (trilinear weight at g of node vox_lane[j]) added to out[j] (per-node test lanes)
+template <int N> DI void addVoxLanes(const DMedium &m, f3 g, real w, real *out) {
+    GridCell c;
+    if (!gridCell(m.res, g, c)) return;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const int v = m.vox_lane[j];
+        if (v < 0) continue;
+        const int dx = v % m.res[0] - c.x, dy = (v / m.res[0]) % m.res[1] - c.y, dz = v / (m.res[0] * m.res[1]) - c.z;
+        if ((unsigned)dx > 1u || (unsigned)dy > 1u || (unsigned)dz > 1u) continue;
+        out[j] += w * ((dx ? c.fx : 1._r - c.fx) * (dy ? c.fy : 1._r - c.fy) * (dz ? c.fz : 1._r - c.fz));
+    }
+}
+
+// heterogeneous.cpp:121-141 — derivative of the optical depth along a segment.
+// The tangent of the grid coordinate under the point's tangents and the volume's rigid
+// motion is affine in t, so the ten points sum the density, its gradient and t times its
+// gradient, and the N lanes are contracted with these sums once, instead of chaining N
+// tangents through every lookup. t counts from tmin, where the motion is taken.
 // With `sc` (adjoint), each of the 10 points also scatters -w * len/10 * scale.
 template <int N>
 DI void intSigT(const DMedium &m, const Dv<N> &o, const Dv<N> &d, real tmin, const Df<N> &tmax, Rng &r, real *out,
                 const ScatterCtx *scx = nullptr) {
-#pragma unroll
-    for (int j = 0; j < N; ++j) out[j] = 0._r;
     const real len = tmax.v - tmin;
-    Df<N> sc = scaleAD<N>(m);
+    const GridRay gr(m, o.val(), d.val());
+    real vox[N], sum = 0._r;
+#pragma unroll
+    for (int j = 0; j < N; ++j) vox[j] = 0._r;
+    f3 g0{0, 0, 0}, g1{0, 0, 0};
     for (int i = 0; i < 10; ++i) {
-        real t = tmin + len * ((i + r.next()) * 0.1_r);
-        Dv<N> x = o + d * Df<N>(t);
-        Df<N> s = sc * lookupDensityAD<N>(m, x);
-        if (scx && &m == scx->pm) scatterDensity(m, x.val(), -scx->w * len * 0.1_r * m.scale, scx->grad);
+        const real u = len * ((i + r.next()) * 0.1_r), t = tmin + u;
+        const f3 g = gr.at(m, t);
+        f3 grad;
+        sum += densityGrad(m, g, grad);
+        g0 = g0 + grad;
+        g1 = g1 + grad * u;
+        if (scx && &m == scx->pm) scatterDensity(m, o.val() + d.val() * t, -scx->w * len * 0.1_r * m.scale, scx->grad);
+        if (m.vox_any) addVoxLanes<N>(m, g, 1._r, vox);
         r.nlk++;
-#pragma unroll
-        for (int j = 0; j < N; ++j) out[j] += s.d[j];
     }
+    const f3 h0 = gradToWorld(m, g0), h1 = gradToWorld(m, g1);
+    const f3 x0 = o.val() + d.val() * tmin, q = x0 - ld3(m.center), dv = d.val();
 #pragma unroll
-    for (int j = 0; j < N; ++j) out[j] *= len * 0.1_r;
+    for (int j = 0; j < N; ++j) {
+        const f3 rot = ld3(m.rot_d[j]);
+        const f3 a = o.grad(j) + d.grad(j) * tmin - cross(rot, q) - ld3(m.trans_d[j]), b = d.grad(j) - cross(rot, dv);
+        out[j] = (m.scale_d[j] * sum + m.scale * (dot(h0, a) + dot(h1, b) + vox[j])) * (len * 0.1_r);
+    }
     if (!tmax.gradZero(EPS)) {
         // The reference steps back Epsilon = 1e-7 from tmax; in fp32 the step is
         // widened to one that is representable at tmax's magnitude.
@@ -505,13 +592,14 @@ DI bool sampleDistance(const DMedium &m, f3 o, f3 d, real tmax, real r0, real r1
     tN = fmax(tN, 0._r);
     tF = fmin(tF, tmax);
     real t = tN;
+    const GridRay gr(m, o, d);
     for (int dep = 0;; ++dep) {
         t -= log(r.next()) * m.maxInvDensity;
         if (t > tF) break;
         if (dep > 10000) break;
-        f3 p = o + d * t;
         r.nlk++;
-        if (r.next() * m.maxDensity < lookupDensity(m, p)) {
+        if (r.next() * m.maxDensity < trilinear(m.density, m.res, gr.at(m, t), 0, 1)) {
+            const f3 p = o + d * t;
             ps = p;
             thr = thr * (m.albedo_grid ? lookupAlbedo(m, p) : ld3(m.albedo));
             return true;
@@ -553,24 +641,32 @@ DI bool sampleDistanceAD(const DMedium &m, const Dv<N> &o, const Dv<N> &d, const
     tF = fmin(tF, tmax.v);
     real t = tN;
     real is[N];
+    const GridRay gr(m, o.val(), d.val());
     for (int dep = 0;; ++dep) {
         t -= log(r.next()) * m.maxInvDensity;
         if (t > tF) break;
         if (dep > 10000) break;
-        Dv<N> p = o + d * Df<N>(t);
-        Df<N> dens = lookupDensityAD<N>(m, p);
+        f3 g;
+        const real dens = densityGrad(m, gr.at(m, t), g);
         r.nlk++;
-        if (r.next() * m.maxDensity < dens.v) {
-            ps = p;
-            Ds<N> alb = m.albedo_grid ? lookupAlbedoAD<N>(m, p) : albedoAD<N>(m);
-            Df<N> sigT = scaleAD<N>(m) * dens;
-            if (scx && &m == scx->pm) scatterDensity(m, p.val(), scx->w / dens.v, scx->grad);
+        if (r.next() * m.maxDensity < dens) {
+            ps = o + d * Df<N>(t);
+            Ds<N> alb = m.albedo_grid ? lookupAlbedoAD<N>(m, ps) : albedoAD<N>(m);
+            if (scx && &m == scx->pm) scatterDensity(m, ps.val(), scx->w / dens, scx->grad);
             intSigT<N>(m, o, d, 0._r, Df<N>(t), r, is, scx);
-            // sigT * (1, -intSigT) / sigT.v
+            // sigT * (1, -intSigT) / sigT.v, sigT = scale * density
             Df<N> w(1._r);
-            real iv = 1.0_r / sigT.v;
+            const real iv = 1.0_r / (m.scale * dens);
+            const f3 h = gradToWorld(m, g), q = ps.val() - ld3(m.center);
+            real vox[N];
 #pragma unroll
-            for (int j = 0; j < N; ++j) w.d[j] = sigT.d[j] * iv - is[j];
+            for (int j = 0; j < N; ++j) vox[j] = 0._r;
+            if (m.vox_any) addVoxLanes<N>(m, toGrid(m, ps.val()), 1._r, vox);
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const f3 a = ps.grad(j) - cross(ld3(m.rot_d[j]), q) - ld3(m.trans_d[j]);
+                w.d[j] = (m.scale_d[j] * dens + m.scale * (dot(h, a) + vox[j])) * iv - is[j];
+            }
             thr = thr * (alb * w);
             return true;
         }
@@ -587,11 +683,12 @@ DI bool sampleDistanceAD(const DMedium &m, const Dv<N> &o, const Dv<N> &d, const
 DI real mediumTransmittance(const DMedium &m, f3 o, f3 d, real tmin, real tmax, Rng &r) {
     if (m.type == MED_HOMOGENEOUS) return exp((tmin - tmax) * m.sigma_t);
     real ret = 1.0_r, t = tmin, inv = 1.0_r / m.maxDensity;
+    const GridRay gr(m, o, d);
     while (ret > EPS) {
         t -= log(r.next()) * m.maxInvDensity;
         if (t > tmax) break;
         r.nlk++;
-        ret *= 1.0_r - lookupDensity(m, o + d * t) * inv;
+        ret *= 1.0_r - trilinear(m.density, m.res, gr.at(m, t), 0, 1) * inv;
     }
     return ret;
 }
