@@ -826,6 +826,17 @@ template <int N> DI Ds<N> specAD(const float *v, const float (*d)[3]) {
 }
 template <int N> DI Df<N> scalarAD(real v, const float *d) { Df<N> r(v); for (int j = 0; j < N; ++j) r.d[j] = d[j]; return r; }
 
+// A diffuse surface without reflectance: it scatters nothing, whatever the directions.
+// Light sources are usually given one (a path that reaches one collects its emission and
+// ends), so its light sample, whose walk costs as much as the segment before it, and its
+// edge samples are left out: they can only add zeros, and nothing draws after them.
+DI bool isBlack(const DBsdf &b) { return b.type == BSDF_DIFFUSE && b.refl[0] == 0.f && b.refl[1] == 0.f && b.refl[2] == 0.f; }
+// ... and none in any tangent lane
+template <int N> DI bool isBlackAD(const DBsdf &b) {
+    bool z = isBlack(b);
+    for (int j = 0; j < N; ++j) z = z && b.refl_d[j][0] == 0.f && b.refl_d[j][1] == 0.f && b.refl_d[j][2] == 0.f;
+    return z;
+}
 // diffuse.cpp:7-38, null.cpp:5-29, phong.cpp:19-95, roughdielectric.cpp:9-206
 // importance: adjoint transport (light tracing); drops the radiance scaling of
 // refraction, roughdielectric.cpp:50,156

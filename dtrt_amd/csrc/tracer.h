@@ -450,6 +450,7 @@ template <int N> struct Tracer {
             if (sh.light_id >= 0 && p.incEmission)
                 p.ret = p.ret + p.thr * emitterEval(S.emitters[sh.light_id], its.gn, its.sn, -p.rd);
             if (p.depth >= p.max_depth) return false;
+            if (isBlack(bsdfOf(S, sh))) return false;   // no light sample counts and no direction follows
             bt = bsdfOf(S, sh).type;
             if (bt != BSDF_NULL) neeSurfaceSetup(its, r2, p.med, max_inter, q);
         }

@@ -72,3 +72,16 @@ def test_rotating_scaled_medium_matches_the_oracle(gpu, oracle):
     b = renders(oracle, d, range(101, 117), **kw)
     assert np.abs(a[:, 1:]).max() > 0
     assert_parity(a, b, 4, what="rotating medium")
+
+
+def test_reflectance_lane_of_a_black_surface_matches_the_oracle(gpu, oracle):
+    """A diffuse surface whose reflectance is zero but has a tangent: its light samples add
+    nothing to the value and all of the lane's derivative, so they are not left out."""
+    d = scenes.ico_surface(nder=2, res=24, spp=16)
+    dref = np.zeros((2, 3), np.float32)
+    dref[1] = (1.0, 0.5, 0.25)
+    d.bsdfs[0] = ("diffuse", (0.0, 0.0, 0.0), dref)
+    a = renders(gpu, d, range(1, 17), sppe=256)
+    b = renders(oracle, d, range(101, 117), sppe=256)
+    assert np.abs(a[:, 2]).max() > 0
+    assert_parity(a, b, 4, what="black surface with a reflectance lane")
