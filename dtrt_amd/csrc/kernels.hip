@@ -43,7 +43,12 @@ DI real edgeAngle(f3 e0, f3 e1, f3 c01, real l0, real l1) {
 __constant__ FrameRot DT_FRAME_ROT;
 
 constexpr int BLOCK = TRACE_BLOCK;
-constexpr int MAX_BLOCK = 256;   // largest work-group size of the AD-path and child kernels
+constexpr int MAX_BLOCK = 256;   // largest work-group size of the AD-path and child kernels that the settings name
+// Work-group of a whole CU's waves at two per SIMD, for trees that fit in LDS once per CU but
+// not once per smaller group (wideGroup). 1,284 triangles, 103 KiB, child kernel per render in
+// double with nodes and triangles read from HBM and from LDS: surface scene 70.3 -> 49.5 ms,
+// dielectric ball on a quad 235 -> 168 ms. Primary-edge samples gain nothing by it.
+constexpr int WIDE_BLOCK = 512;
 // Work-group size of the primal path and particle kernels: four waves, so that at their
 // occupancy a small scene's tree fits in LDS beside the traversal stacks (treeLdsFor).
 constexpr int PRIMAL_BLOCK = 256;
@@ -1061,7 +1066,7 @@ DI void scatterFinished(const RenderParams &P, const char *q, real *acc, real *a
 // iteration; a lane whose path has ended takes the next queued record (one atomic
 // per wave on qnext), so the lanes of a wave stay busy until the queue is drained.
 template <int N>
-__global__ __launch_bounds__(MAX_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
+__global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
                                                     unsigned *qnext, real *acc, real *acc_pe, unsigned long long *work) {
     Tracer<N> T(S);
     T.useLdsTree(P);
@@ -1126,7 +1131,7 @@ __global__ __launch_bounds__(MAX_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(DS
 // Persistent drain of CHILD_PATH records (the surface-only integrators' sub-paths,
 // path.cpp:11-61 from the record's origin and direction), as k_children.
 template <int N>
-__global__ __launch_bounds__(MAX_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_path(DScene S, RenderParams P, const char *q,
+__global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_path(DScene S, RenderParams P, const char *q,
                                                                             const unsigned *qcount, unsigned *qnext,
                                                                             real *acc, real *acc_pe,
                                                                             unsigned long long *work) {
@@ -1449,6 +1454,16 @@ template <class K> static size_t treeLdsFor(K kern, unsigned blk, const DScene &
     return tb;
 }
 
+// The work-group size of a launch of `kern` whose default is `blk`: WIDE_BLOCK where only that
+// many waves, sharing one copy, leave room for the whole tree.
+template <class K> static unsigned wideGroup(K kern, unsigned blk, const DScene &S, const RenderParams &P) {
+    RenderParams a = P, b = P;
+    (void)treeLdsFor(kern, blk, S, a, false);
+    if (a.lds_tris) return blk;
+    (void)treeLdsFor(kern, WIDE_BLOCK, S, b, false);
+    return b.lds_tris ? (unsigned)WIDE_BLOCK : blk;
+}
+
 template <class Sym> static hipError_t setRotation(const Sym &sym, const double *m9) {
     FrameRot r;
     for (int i = 0; i < 9; ++i) r.m[i] = (real)m9[i];
@@ -1524,15 +1539,17 @@ template <int N> void WidthOps<N>::launchAdStages(const DScene &S, const RenderP
 }
 template <int N> void WidthOps<N>::launchChildren(const DScene &S, const RenderParams &P, const char *q, unsigned *qc,
                                             real *acc, real *acc_pe, unsigned long long *wk, unsigned grid, hipStream_t sm) {
-    const unsigned blk = blockOr64(P.child_block);   // grid: blocks of `blk` threads
+    const unsigned dflt = blockOr64(P.child_block);   // grid: blocks of that many threads
     RenderParams Pl = P;
     if (P.ad_kind == AD_VOLPATH) {
+        const unsigned blk = wideGroup(k_children<N>, dflt, S, P);
         const size_t tl = treeLdsFor(k_children<N>, blk, S, Pl, treePrefixInLds<N>());
-        hipLaunchKernelGGL(k_children<N>, dim3(grid), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, q, qc, qc + 2, acc, acc_pe,
+        hipLaunchKernelGGL(k_children<N>, dim3(std::max(1u, grid * dflt / blk)), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, q, qc, qc + 2, acc, acc_pe,
                            wk);
     } else {
+        const unsigned blk = wideGroup(k_children_path<N>, dflt, S, P);
         const size_t tl = treeLdsFor(k_children_path<N>, blk, S, Pl, treePrefixInLds<N>());
-        hipLaunchKernelGGL(k_children_path<N>, dim3(grid), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, q, qc, qc + 2, acc,
+        hipLaunchKernelGGL(k_children_path<N>, dim3(std::max(1u, grid * dflt / blk)), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, q, qc, qc + 2, acc,
                            acc_pe, wk);
     }
 }

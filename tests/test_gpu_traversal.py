@@ -70,3 +70,23 @@ def test_smallest_trees_render_the_same_from_lds_and_hbm(gpu, ntri):
     hbm = scenes.render_primal(gpu, d, seed=5, scene=sc)
     assert lds.max() == pytest.approx(3.0, rel=1e-6)
     assert np.allclose(lds, hbm, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("subdiv,rtol", [(3, 1e-5), (4, 1e-5)])
+def test_middle_trees_render_the_same_from_lds_and_hbm(gpu, subdiv, rtol):
+    """1,280 triangles fit in LDS once per compute unit, beside the stacks of one work-group of
+    eight waves; 5,120 do not fit at all. Value and tangent images, child paths included,
+    are the same from either memory (double sums in another order, rounded to float)."""
+    d = scenes.ico_surface(nder=3, res=40, spp=32)
+    v, f = scenes.icosphere(subdiv, 0.5, (0, 0.5, 0))
+    vel = np.zeros((3, len(v), 3), np.float32)
+    vel[0, :, 0] = vel[1, :, 1] = vel[2, :, 2] = 1.0
+    d.shapes[1] = scenes.ShapeDesc(v, f, bsdf_id=1, velocities=vel)
+    sc = scenes.instantiate(gpu, d)
+    lds = scenes.render(gpu, d, seed=3, scene=sc, sppe=256).astype(np.float64)
+    assert gpu.render_stats(sc)["children"] > 0
+    gpu.set_tree_in_hbm(sc, True)
+    hbm = scenes.render(gpu, d, seed=3, scene=sc, sppe=256).astype(np.float64)
+    for lane in range(4):
+        assert np.abs(lds[lane]).max() > 0
+        assert np.allclose(lds[lane], hbm[lane], rtol=rtol, atol=rtol * 1e-2 * np.abs(lds[lane]).max()), lane
