@@ -171,14 +171,20 @@ template <int N> HDI Ds<N> &operator+=(Ds<N> &a, const Ds<N> &b) { a = a + b; re
 // 1, 2, 3", SC'11): counter-based, so any draw of any path can be regenerated from
 // (key, path id, stream, index) — the property adjoint path replay relies on.
 struct u4 { uint32_t a, b, c, d; };
-HDI uint32_t mulhi32(uint32_t a, uint32_t b) { return (uint32_t)(((uint64_t)a * b) >> 32); }
-HDI u4 philox4x32_10(u4 ctr, uint32_t k0, uint32_t k1) {
+// Both words of a 32 x 32 bit product in one instruction: two of these per round cost half of
+// the two high and two low products that the compiler makes of the plain expression
+// (benchmark scene, child kernel per render: 194 -> 189 ms).
+DI uint64_t mulWide(uint32_t a, uint32_t b) {
+    uint64_t p;
+    asm("v_mad_u64_u32 %0, vcc, %1, %2, 0" : "=v"(p) : "v"(a), "s"(b) : "vcc");
+    return p;
+}
+DI u4 philox4x32_10(u4 ctr, uint32_t k0, uint32_t k1) {
     const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
 #pragma unroll
     for (int r = 0; r < 10; ++r) {
-        uint32_t hi0 = mulhi32(M0, ctr.a), lo0 = M0 * ctr.a;
-        uint32_t hi1 = mulhi32(M1, ctr.c), lo1 = M1 * ctr.c;
-        ctr = u4{hi1 ^ ctr.b ^ k0, lo1, hi0 ^ ctr.d ^ k1, lo0};
+        const uint64_t p0 = mulWide(ctr.a, M0), p1 = mulWide(ctr.c, M1);
+        ctr = u4{(uint32_t)(p1 >> 32) ^ ctr.b ^ k0, (uint32_t)p1, (uint32_t)(p0 >> 32) ^ ctr.d ^ k1, (uint32_t)p0};
         k0 += W0;
         k1 += W1;
     }
@@ -193,7 +199,7 @@ struct Rng {
     uint32_t b0, b1, b2, b3;
     int pos;
     uint32_t nlk;   // density-grid lookups made along this stream's path (work counter)
-    HDI void init(uint64_t seed, uint64_t stream) {
+    DI void init(uint64_t seed, uint64_t stream) {
         nlk = 0;
         k0 = (uint32_t)seed;
         k1 = (uint32_t)(seed >> 32) ^ 0x5bd1e995u;
@@ -202,7 +208,7 @@ struct Rng {
         blk = 0;
         pos = 4;
     }
-    HDI real next() {
+    DI real next() {
         if (pos == 4) {
             u4 o = philox4x32_10(u4{s0, s1, blk++, 0x9e3779b9u}, k0, k1);
             b0 = o.a; b1 = o.b; b2 = o.c; b3 = o.d;
