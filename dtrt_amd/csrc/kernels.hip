@@ -1062,16 +1062,26 @@ DI void scatterFinished(const RenderParams &P, const char *q, real *acc, real *a
     }
 }
 
+// Lanes of a wave that take records when a launch drains n of them: an even share of a
+// short queue for every wave, since a wave's time grows with the lanes that diverge in it
+// (a 32x32 render of 4 samples per pixel, 17K sub-paths: child kernels 0.95 -> 0.39 ms).
+DI int lanesToUse(unsigned n) {
+    const unsigned waves = gridDim.x * (blockDim.x / 64), even = (n + waves - 1) / waves;
+    return even >= 64 ? 64 : even < 4 ? 4 : (int)even;
+}
+
 // Persistent: each lane holds one primal sub-path and advances it one bounce per
 // iteration; a lane whose path has ended takes the next queued record (one atomic
 // per wave on qnext), so the lanes of a wave stay busy until the queue is drained.
 template <int N>
 __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
                                                     unsigned *qnext, real *acc, real *acc_pe, unsigned long long *work) {
+    const unsigned n = min(*qcount, P.qcap);
+    if (blockIdx.x >= n) return;   // each block before this one has a record
     Tracer<N> T(S);
     T.useLdsTree(P);
-    const unsigned n = min(*qcount, P.qcap);
     const int lane = threadIdx.x & 63;
+    const bool use = lane < lanesToUse(n);
     uint32_t nlk = 0;
     bool alive = false, exhausted = false;
     unsigned rec = 0;
@@ -1082,7 +1092,7 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(D
         bool fin = false;
         f3 Lv{0, 0, 0};
         if (!exhausted) {
-            const uint64_t need = __ballot(!alive);
+            const uint64_t need = __ballot(use && !alive);
             if (need) {
                 const int lead = __ffsll((unsigned long long)need) - 1;
                 unsigned base = 0;
@@ -1090,7 +1100,7 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(D
                 base = __shfl(base, lead);
                 if (base + __popcll(need) >= n) exhausted = true;
                 const unsigned my = base + (unsigned)__popcll(need & ((1ull << lane) - 1ull));
-                if (!alive && my < n) {
+                if (use && !alive && my < n) {
                     rec = my;
                     const ChildHdr h = *reinterpret_cast<const ChildHdr *>(q + (size_t)rec * P.rec_stride);
                     r.init(S.views[h.view].seed ^ 0x6a09e667f3bcc909ull, ((uint64_t)h.key_hi << 32) | h.key_lo);
@@ -1135,10 +1145,12 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_p
                                                                             const unsigned *qcount, unsigned *qnext,
                                                                             real *acc, real *acc_pe,
                                                                             unsigned long long *work) {
+    const unsigned n = min(*qcount, P.qcap);
+    if (blockIdx.x >= n) return;   // each block before this one has a record
     Tracer<N> T(S);
     T.useLdsTree(P);
-    const unsigned n = min(*qcount, P.qcap);
     const int lane = threadIdx.x & 63;
+    const bool use = lane < lanesToUse(n);
     uint32_t nlk = 0;
     bool alive = false, exhausted = false;
     unsigned rec = 0;
@@ -1148,7 +1160,7 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_p
         bool fin = false;
         f3 Lv{0, 0, 0};
         if (!exhausted) {
-            const uint64_t need = __ballot(!alive);
+            const uint64_t need = __ballot(use && !alive);
             if (need) {
                 const int lead = __ffsll((unsigned long long)need) - 1;
                 unsigned base = 0;
@@ -1156,7 +1168,7 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_p
                 base = __shfl(base, lead);
                 if (base + __popcll(need) >= n) exhausted = true;
                 const unsigned my = base + (unsigned)__popcll(need & ((1ull << lane) - 1ull));
-                if (!alive && my < n) {
+                if (use && !alive && my < n) {
                     rec = my;
                     const ChildHdr h = *reinterpret_cast<const ChildHdr *>(q + (size_t)rec * P.rec_stride);
                     r.init(S.views[h.view].seed ^ 0x6a09e667f3bcc909ull, ((uint64_t)h.key_hi << 32) | h.key_lo);
@@ -1539,19 +1551,18 @@ template <int N> void WidthOps<N>::launchAdStages(const DScene &S, const RenderP
 }
 template <int N> void WidthOps<N>::launchChildren(const DScene &S, const RenderParams &P, const char *q, unsigned *qc,
                                             real *acc, real *acc_pe, unsigned long long *wk, unsigned grid, hipStream_t sm) {
-    const unsigned dflt = blockOr64(P.child_block);   // grid: blocks of that many threads
+    // grid: the most blocks of the default size; no more than the device holds at once are
+    // launched, since each drains the queue until it is empty
+    const unsigned dflt = blockOr64(P.child_block);
     RenderParams Pl = P;
-    if (P.ad_kind == AD_VOLPATH) {
-        const unsigned blk = wideGroup(k_children<N>, dflt, S, P);
-        const size_t tl = treeLdsFor(k_children<N>, blk, S, Pl, treePrefixInLds<N>());
-        hipLaunchKernelGGL(k_children<N>, dim3(std::max(1u, grid * dflt / blk)), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, q, qc, qc + 2, acc, acc_pe,
-                           wk);
-    } else {
-        const unsigned blk = wideGroup(k_children_path<N>, dflt, S, P);
-        const size_t tl = treeLdsFor(k_children_path<N>, blk, S, Pl, treePrefixInLds<N>());
-        hipLaunchKernelGGL(k_children_path<N>, dim3(std::max(1u, grid * dflt / blk)), dim3(blk), traceLds(blk, S.stack_depth) + tl, sm, S, Pl, q, qc, qc + 2, acc,
-                           acc_pe, wk);
-    }
+    auto launch = [&](auto kern) {
+        const unsigned blk = wideGroup(kern, dflt, S, P);
+        const size_t lds = traceLds(blk, S.stack_depth) + treeLdsFor(kern, blk, S, Pl, treePrefixInLds<N>());
+        const unsigned nb = std::min(std::max(1u, grid * dflt / blk), residentBlocks(kern, blk, lds));
+        hipLaunchKernelGGL(kern, dim3(nb), dim3(blk), lds, sm, S, Pl, q, qc, qc + 2, acc, acc_pe, wk);
+    };
+    if (P.ad_kind == AD_VOLPATH) launch(k_children<N>);
+    else launch(k_children_path<N>);
 }
 template <int N> void WidthOps<N>::launchPrimary(const DScene &S, const RenderParams &P, int view, uint64_t s0, uint64_t n,
                                            uint64_t total, char *q, unsigned *qc, unsigned *st, unsigned long long *wk,
