@@ -1,12 +1,15 @@
 // VolPathTracerAD samples in stages: the paths of a batch of samples advance one bounce
 // per launch, with their state in HBM between launches.
 //
-//  k_ad_bounce<N>   one bounce (ad_bounce.inc) of every path still alive, the continuation
-//                   walk that the last bounce handed over first; the first launch of a
-//                   batch starts the samples at their camera rays
+//  k_ad_bounce<N>   one bounce (adBounce) of every path still alive, the continuation walk
+//                   that the last bounce handed over first; the first launch of a batch
+//                   starts the samples at their camera rays
 //  k_ad_edges<N>    the edge term (edgeTerm) of the bounces that have one
 //  k_ad_finish<N>   the samples' radiance into the accumulators, the samples whose pushes
 //                   overflowed the queue into the replay list
+//  k_adj_list<N>, k_adj_bounce<N>
+//                   the density adjoint: which samples take part, and the bounces of the
+//                   replay that scatters the derivative of every contribution
 //
 // Included by kernels.hip.
 #pragma once
@@ -21,6 +24,7 @@ template <int N> struct AdSlots {
     enum Real { RO = 0, RD = 3 * (N + 1), BETA = 6 * (N + 1), L = 9 * (N + 1), CPDF = 12 * (N + 1), ETHR, EBETA = ETHR + 3,
                 EWI = EBETA + 3, EGN = EWI + 3, ESN = EGN + 3, REALS = ESN + 3 };
     enum Word { PIX = 0, VIEW, FLAGS, FACE, RBLK, RPOS, RB0, RB1, RB2, RB3, CHILD, SKIP, FAILED, EFLAGS, EFACE, WORDS };
+    static constexpr size_t BYTES = REALS * sizeof(real) + WORDS * 4;
     static_assert(REALS == adSlotReals(N) && WORDS == AD_SLOT_WORDS, "adSlotBytes sizes this layout");
     static constexpr uint32_t RD_CONST = 1u << 31;   // FLAGS: rd has no tangents (none are stored)
     DI real &r(int k, uint32_t slot) const { return f[(size_t)k * n + slot]; }
@@ -72,9 +76,10 @@ struct AdBatch {
     uint32_t m;                  // samples of the batch, <= n
     uint64_t s0;                 // first sample (replay == nullptr)
     const uint4 *replay;         // or the batch's entries {sid lo, sid hi, children delivered, 0}
-    const uint32_t *in;          // slots alive at the start of the bounce (nullptr: all m, started here)
+    int start;                   // the bounce starts its paths at their camera rays
+    const uint32_t *in;          // slots alive at the start of the bounce (nullptr: all m)
     uint32_t *out, *edges;       // slots alive after it; slots with an edge term
-    uint32_t *cnt;               // [0] length of in, [1] consumed, [2] length of edges, [3] consumed, [4] length of out
+    uint32_t *cnt;               // AD_CNT words apart: length of in, consumed, length of edges, consumed, length of out
 };
 template <int N> DI AdSlots<N> slotsOf(const AdBatch &B) {
     AdSlots<N> a;
@@ -83,29 +88,6 @@ template <int N> DI AdSlots<N> slotsOf(const AdBatch &B) {
     a.w = reinterpret_cast<uint32_t *>(a.f + (size_t)AdSlots<N>::REALS * B.n);
     return a;
 }
-
-// Where a bounce's edge term is written for k_ad_edges (AD_EDGE_DEFERRED of ad_bounce.inc).
-template <int N> struct AdEdgeOut {
-    const AdSlots<N> &a;
-    uint32_t slot;
-    bool set;
-    DI void put(bool vol, const Dv<N> &x, const Hit &its0, f3 rdin, f3 thrv, f3 betav, int med, int depth) {
-        using A = AdSlots<N>;
-        set = true;
-        a.stv(A::RO, slot, x);   // also the next ray's origin
-        a.st(A::ETHR, slot, thrv);
-        a.st(A::EBETA, slot, betav);
-        a.u(A::EFLAGS, slot) = (vol ? 1u : 0u) | (uint32_t)depth << 1 | (uint32_t)(med + 1) << 9;
-        if (vol) {
-            a.st(A::EWI, slot, rdin);
-        } else {
-            a.u(A::EFACE, slot) = (uint32_t)its0.face;
-            a.st(A::EWI, slot, its0.wi);
-            a.st(A::EGN, slot, its0.gn);
-            a.st(A::ESN, slot, its0.sn);
-        }
-    }
-};
 
 // A wave's share of a list of `n` items. It takes a full wave's at a time while there are
 // more than the launch's waves can hold, else an even share, so that a short list (a small
@@ -144,95 +126,374 @@ DI void appendSlots(bool put, uint32_t slot, uint32_t *list, uint32_t *len) {
     if (put) list[base + (uint32_t)__popcll(m & __lanemask_lt())] = slot;
 }
 
+// State of one AD path between bounces, but for its throughput and radiance, which stay in
+// its slot until they are needed.
+template <int N> struct AdState {
+    Dv<N> ro, rd;
+    int med, depth, mode;
+    // The walk along (ro, rd) to run first: 1 first hit only from a surface, 2 emitter walk,
+    // 3 the camera ray's first hit (from 0); walk_add: its emitter term counts, with MIS
+    // partner pdf walk_cpdf.
+    int walk;
+    bool walk_surf, walk_add;
+    real walk_cpdf;
+};
+// Passes over a path: FORWARD adds its radiance with tangents into its slot; SCATTER replays
+// it from the same stream and adds the reverse-mode density derivative of every
+// contribution into grad (AdjCtx).
+enum class AdPass { FORWARD, SCATTER };
+struct AdjCtx {
+    double *grad;        // d loss / d node density of the grid of *pm (accumulated)
+    const DMedium *pm;
+    f3 adj;              // d loss / d pixel value of this sample (already / spp)
+    f3 Ltot;             // the sample's radiance
+};
+
+// One bounce of the dual-number estimator LiAD (volpathAD.cpp:145-620) for the path of `slot`.
+// alive, edge: what follows.
+//
+// The path carries only the face its ray (ro, rd) hits: the hit record with its tangents is
+// recomputed from the face and the dual ray, by the same refinement that produced it
+// (shape.cpp:210-252). The two kinds of event, a scattering in the medium
+// (volpathAD.cpp:171-305) and a surface hit (:306-616), run the same steps in the same
+// order: the light sample (NEE), the edge term, the continuation's walk to the next hit.
+// Each is set up per kind and then runs once for both, so the lanes of a wave on either kind
+// of event share one shadow walk, one edge term and one continuation walk. The edge term
+// is left to k_ad_edges and the continuation's walk to the next launch.
+//
+// What bounds it is the size of a dual-number path, which spills. The draws of the light
+// sample and of the continuation all come before the shadow walk's, so the continuation
+// is sampled and stored before that walk, and throughput and radiance are read and
+// written where they are used: the hit record, the throughput and the radiance are not
+// live across it.
+template <int N, AdPass A>
+DI void adBounce(Tracer<N> &T, const RenderParams &P, const AdSlots<N> &a, uint32_t slot, Rng &r, AdState<N> &st, Pusher &u,
+                 unsigned *stats, const AdjCtx *ac, bool &alive, bool &edge) {
+    using AS = AdSlots<N>;
+    const DScene &S = T.S;
+    alive = edge = false;
+    Dv<N> ro = st.ro;
+    const Dv<N> &rd = st.rd;
+    const int med = st.med, depth = st.depth, mode = st.mode;
+    auto addL = [&](const Ds<N> &c) {
+        if constexpr (A == AdPass::FORWARD) a.sts(AS::L, slot, a.lds(AS::L, slot) + c);
+        else a.st(AS::L, slot, a.ld(AS::L, slot) + c.val());
+    };
+    int hface = -1;
+    {   // the walk the last bounce handed over, or the camera ray's first hit
+        real pdf_nee = 0._r;
+        Rng rs;   // stream position before the walk (scatter pass only)
+        if constexpr (A == AdPass::SCATTER) rs = r;
+        const Ds<N> att = T.lookForEmitterAD(ro, rd, st.walk_surf, r, med, depth, hface, pdf_nee, nullptr, nullptr, nullptr,
+                                             st.walk != 2);
+        if (st.walk_add && !att.isZero(EPS)) {
+            const Ds<N> c = a.lds(AS::BETA, slot) * (att * misPower(st.walk_cpdf, pdf_nee));
+            addL(c);
+            if constexpr (A == AdPass::SCATTER) {
+                ScatterCtx sc{ac->grad, ac->pm, dot(ac->adj, c.val())};
+                Rng r2 = rs;
+                int f2;
+                real pdf2;
+                T.lookForEmitterAD(ro, rd, st.walk_surf, r2, med, depth, f2, pdf2, nullptr, nullptr, &sc);
+            }
+        }
+        if (st.walk == 3 && hface < 0) return;
+    }
+    HitAD<N> its;
+    if (hface >= 0) refineHitAD<N>(S, hface, ro, rd, its);
+    else its.t = Df<N>(FINF);
+    const real r1a = r.next(), r1b = r.next();
+    const real r2[4] = {r.next(), r.next(), r.next(), r.next()};
+    const real r3[3] = {r.next(), r.next(), r.next()};
+    Ds<N> thr(f3{1, 1, 1});
+    bool vol = false;
+    if (med >= 0) {
+        Dv<N> ps;
+        ScatterCtx fs{nullptr, nullptr, 0._r};
+        const ScatterCtx *fsp = nullptr;
+        if constexpr (A == AdPass::SCATTER) {   // free flight weighs everything from here on
+            fs = ScatterCtx{ac->grad, ac->pm, dot(ac->adj, ac->Ltot - a.ld(AS::L, slot))};
+            fsp = &fs;
+        }
+        vol = sampleDistanceAD<N>(S.media[med], ro, rd, its.t, r1a, r1b, r, ps, thr, fsp);
+        if (vol) ro = ps;
+    }
+    const f3 rdin = rd.val();
+    typename Tracer<N>::ShadowAD q;
+    q.live = false;
+    Ds<N> f;                          // the light sample's weight but for its radiance and MIS weight
+    real fpdf = 0._r;                 // its MIS partner pdf
+    bool fadd = true, cont = false, first_only = false;
+    f3 nd{0, 0, 0};                   // the continuation's direction (through a null surface: rd)
+    real cpdf = 1._r;
+    int med1 = med;
+    Ds<N> beta = a.lds(AS::BETA, slot);
+    if (vol) {
+        if (depth == 0 || thr.isZero(EPS)) return;
+        const DPhase &ph = S.phases[S.media[med].phase_id];
+        if (mode & 8) T.neePointADSetup(ro, r2, med, depth - 1, q);   // volume NEE with tangents
+        const Ds<N> bt = beta * thr;
+        if (q.live) {
+            const Df<N> pv = phaseEvalAD<N>(ph, -rd, q.d);
+            fadd = pv.v > EPS;
+            f = bt * pv;
+            fpdf = phaseEval(ph, -rdin, q.d);
+        }
+        if (P.sppse > 0 && (mode & 32) && S.edges_valid) {   // volume edges (volpathAD.cpp:207-305)
+            edge = true;
+            a.st(AS::ETHR, slot, thr.val());
+            a.st(AS::EBETA, slot, beta.val());
+            a.st(AS::EWI, slot, rdin);
+        }
+        nd = phaseSample(ph, -rdin, r3[0], r3[1]);   // volpathAD.cpp:250-268
+        const Df<N> pv = phaseSampleWeightAD<N>(ph, -rd, nd);
+        cont = pv.v > EPS;
+        if (cont) a.sts(AS::BETA, slot, bt * pv);
+        cpdf = phaseEval(ph, -nd, nd);
+    } else {
+        if (its.face < 0 || thr.isZero(EPS)) return;
+        const DShape &sh = shapeOf(S, its.face);
+        if (isTransition(sh) && targetMedium(sh, its.gn.val(), -rdin) != med) {
+            atomicAdd(stats + STAT_MED_INCONSISTENT, 1u);
+            return;
+        }
+        if (sh.light_id >= 0 && (mode & 1)) addL(beta * (thr * emitterEvalAD<N>(S.emitters[sh.light_id], its, -rd)));
+        if (depth == 0) return;
+        const DBsdf &b = bsdfOf(S, sh);
+        const bool isnull = b.type == BSDF_NULL;
+        const Hit its0 = its.val();
+        // Lins boundary term (volpathAD.cpp:321-467): queued as primal sub-paths
+        if (A == AdPass::FORWARD && med >= 0 && !its.t.gradZero(EPS) && (mode & 16)) {
+            int ns = min(max((int)(P.ddist * its.t.gradAbsMax()), 1), 100);
+            f3 n = dot(its0.gn, rdin) < 0._r ? -its0.gn : its0.gn;
+            f3 sgs = sigS(S.media[med], its0.p - n * SHADOW_EPS);
+            f3 base = beta.val() * thr.val() * sgs * (1.0_r / ns);
+            real W[N * 3];
+#pragma unroll
+            for (int j = 0; j < N; ++j) { W[3 * j] = base.x * its.t.d[j]; W[3 * j + 1] = base.y * its.t.d[j]; W[3 * j + 2] = base.z * its.t.d[j]; }
+            ChildHdr h;
+            h.org[0] = its0.p.x; h.org[1] = its0.p.y; h.org[2] = its0.p.z;
+            h.dir[0] = rdin.x; h.dir[1] = rdin.y; h.dir[2] = rdin.z;
+            h.meta = (isnull ? CHILD_LINS_NULL : CHILD_LINS_SURF) | (depth << 4) | ((med + 1) << 12);
+            h.face = its0.face;
+            h.gn[0] = its0.gn.x; h.gn[1] = its0.gn.y; h.gn[2] = its0.gn.z;
+            h.sn[0] = its0.sn.x; h.sn[1] = its0.sn.y; h.sn[2] = its0.sn.z;
+            for (int s = 0; s < ns; ++s) push(P, u, h, W, N * 3);
+        }
+        if (isBlackAD<N>(b)) return;   // no light or edge sample counts and no direction follows
+        ro = its.p;
+        if (isnull) {
+            nd = rdin;   // toWorld(-wi) == incoming direction, tangents included (rd)
+            cont = first_only = true;
+            a.sts(AS::BETA, slot, beta * thr);
+        } else {
+            if (mode & 2) T.neeSurfaceADSetup(its, r2, med, depth - 1, q);   // surface NEE with tangents
+            const Ds<N> bt = beta * thr;
+            const FrameAD<N> shf(its.sn);
+            if (q.live) {
+                const Dv<N> woL = shf.toLocal(Dv<N>(q.d));
+                f = bt * bsdfEvalAD<N>(b, its.wi, woL);
+                fpdf = bsdfPdf(b, its0.wi, woL.val());
+            }
+            if (P.sppse > 0 && (mode & 4) && S.edges_valid) {   // interface edges (volpathAD.cpp:513-616)
+                edge = true;
+                a.st(AS::ETHR, slot, thr.val());
+                a.st(AS::EBETA, slot, beta.val());
+                a.u(AS::EFACE, slot) = (uint32_t)its0.face;
+                a.st(AS::EWI, slot, its0.wi);
+                a.st(AS::EGN, slot, its0.gn);
+                a.st(AS::ESN, slot, its0.sn);
+            }
+            f3 wo0;   // bsdf.cpp:11-21; null.cpp:18-23
+            const f3 w0 = bsdfSample(b, its0.wi, r3[0], r3[1], r3[2], wo0, cpdf);
+            if (!allZero(w0, EPS) && cpdf > EPS) {
+                nd = shf.val().toWorld(wo0);
+                const Ds<N> bw = bsdfEvalAD<N>(b, its.wi, shf.toLocal(Dv<N>(nd))) * (1.0_r / cpdf);
+                cont = !bw.isZero(EPS);
+                if (cont) a.sts(AS::BETA, slot, bt * bw);
+            }
+        }
+        if (cont) med1 = isTransition(sh) ? targetMedium(sh, its0.gn, nd) : med;
+    }
+    if (edge) a.u(AS::EFLAGS, slot) = (vol ? 1u : 0u) | (uint32_t)depth << 1 | (uint32_t)(med + 1) << 9;
+    if (edge || cont) a.stv(AS::RO, slot, ro);   // the edge term's vertex and the next ray's origin
+    if (cont) {
+        const int mode1 = first_only ? mode : mode & ~1;
+        const bool addc = !first_only && (mode & (vol ? 8 : 2)) != 0;
+        const bool keep = first_only && !rd.gradZero(0._r);   // the direction's tangents go on
+        if (keep) a.stv(AS::RD, slot, rd);
+        else a.st(AS::RD, slot, nd);
+        a.r(AS::CPDF, slot) = cpdf;
+        a.u(AS::FLAGS, slot) = (uint32_t)(med1 + 1) | (uint32_t)(depth - 1) << 8 | (uint32_t)mode1 << 16 |
+                               (first_only ? 1u : 2u) << 22 | (vol ? 0u : 1u << 24) | (addc ? 1u << 25 : 0u) |
+                               (keep ? 0u : AS::RD_CONST);
+        alive = mode1 != 0;
+    }
+    if (q.live) {   // one shadow walk for both kinds of event
+        real pdf_nee = 0._r;
+        Rng rs;   // stream position before the walk (scatter pass only)
+        if constexpr (A == AdPass::SCATTER) rs = r;
+        const Ds<N> value = T.neeWalkAD(q, r, pdf_nee);
+        if (fadd && !value.isZero(EPS)) {
+            const Ds<N> c = f * value * misPower(pdf_nee, fpdf);
+            addL(c);
+            if constexpr (A == AdPass::SCATTER) {   // the shadow walk weighs this term only
+                ScatterCtx sc{ac->grad, ac->pm, dot(ac->adj, c.val())};
+                Rng r2w = rs;
+                real pdf2;
+                T.neeWalkAD(q, r2w, pdf2, &sc);
+            }
+        }
+    }
+}
+
+// The path of `slot` at the start of a bounce: its camera ray (B.start) or its stored state.
+// False when it has nothing to do.
+template <int N>
+DI bool adLoad(const DScene &S, const RenderParams &P, const AdBatch &B, const AdSlots<N> &a, uint32_t slot, Rng &r, AdState<N> &st,
+               Pusher &u) {
+    using A = AdSlots<N>;
+    uint64_t sid = B.s0 + slot;
+    if (B.replay) {
+        const uint4 e = B.replay[slot];
+        sid = (uint64_t)e.x | ((uint64_t)e.y << 32);
+        u.skip = e.z;
+    }
+    u.view = B.start ? viewOf(S, sid) : (int)a.u(A::VIEW, slot);
+    const DView &vw = S.views[u.view];
+    const uint64_t ls = sid - vw.s0;   // sample index within the view: keys its random stream
+    u.key = (ls + 1) << 20;
+    if (B.start) {
+        const int pixel = (int)(ls / (uint64_t)vw.spp);
+        u.gpix = vw.pix0 + pixel;
+        a.u(A::PIX, slot) = (uint32_t)u.gpix;
+        a.u(A::VIEW, slot) = (uint32_t)u.view;
+        a.u(A::SKIP, slot) = u.skip;
+        a.sts(A::BETA, slot, Ds<N>(f3{1, 1, 1}));
+        a.sts(A::L, slot, Ds<N>());
+        r.init(vw.seed, ls);
+        adCameraRay<N>(vw, r, pixel, st.ro, st.rd);
+        st.walk = 3;
+        st.walk_surf = st.walk_add = false;
+        st.walk_cpdf = 0._r;
+        st.med = vw.cam.med_id;
+        st.depth = P.max_bounces;
+        st.mode = P.mode;
+        return st.mode != 0;
+    }
+    u.gpix = (int)a.u(A::PIX, slot);
+    u.child = a.u(A::CHILD, slot);
+    u.failed_at = a.u(A::FAILED, slot);
+    a.ldRng(slot, vw.seed, ls, r);
+    const uint32_t fl = a.u(A::FLAGS, slot);
+    st.med = (int)(fl & 255u) - 1;
+    st.depth = (int)(fl >> 8 & 255u);
+    st.mode = (int)(fl >> 16 & 63u);
+    st.walk = (int)(fl >> 22 & 3u);
+    st.walk_surf = (fl >> 24 & 1u) != 0;
+    st.walk_add = (fl >> 25 & 1u) != 0;
+    st.walk_cpdf = a.r(A::CPDF, slot);
+    st.ro = a.ldv(A::RO, slot);
+    st.rd = fl & A::RD_CONST ? Dv<N>(a.ld(A::RD, slot)) : a.ldv(A::RD, slot);
+    return true;
+}
+
 template <int N>
 __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_ad_bounce(DScene S, RenderParams P, AdBatch B, char *q,
                                                                              unsigned *qcount, unsigned *stats,
                                                                              unsigned long long *work) {
     using A = AdSlots<N>;
     const A a = slotsOf<N>(B);
-    const bool first = B.in == nullptr;
-    ListShare share(B.cnt + 1, first ? B.m : B.cnt[0]);
+    ListShare share(B.cnt + AD_CNT, B.in ? B.cnt[0] : B.m);
     if (share.idleBlock()) return;
     Tracer<N> T(S);
     T.useLdsTree(P);
     uint32_t nlk = 0;
     for (; share.more(); share.next()) {
-        uint32_t li;
-        const bool active = share.item(li);
+        uint32_t li, slot = 0;
         bool alive = false, edge = false;
-        uint32_t slot = 0;
-        if (active) {
-            slot = first ? li : B.in[li];
+        if (share.item(li)) {
+            slot = B.in ? B.in[li] : li;
             AdState<N> st;
             Rng r;
             Pusher u{q, qcount, 0, 0, 0, 0, 0, Pusher::NO_FAIL};
-            uint64_t sid = B.s0 + slot;
-            if (B.replay) {
-                const uint4 e = B.replay[slot];
-                sid = (uint64_t)e.x | ((uint64_t)e.y << 32);
-                u.skip = e.z;
-            }
-            if (first) {
-                u.view = viewOf(S, sid);
-                const DView &vw = S.views[u.view];
-                const uint64_t ls = sid - vw.s0;   // sample index within the view: keys its random stream
-                const int pixel = (int)(ls / (uint64_t)vw.spp);
-                u.gpix = vw.pix0 + pixel;
-                u.key = (ls + 1) << 20;
-                r.init(vw.seed, ls);
-                alive = adBegin<N>(P, vw, r, pixel, st);
-                a.u(A::PIX, slot) = (uint32_t)u.gpix;
-                a.u(A::VIEW, slot) = (uint32_t)u.view;
-                a.u(A::SKIP, slot) = u.skip;
-            } else {
-                u.gpix = (int)a.u(A::PIX, slot);
-                u.view = (int)a.u(A::VIEW, slot);
-                const DView &vw = S.views[u.view];
-                const uint64_t ls = sid - vw.s0;
-                u.key = (ls + 1) << 20;
-                u.child = a.u(A::CHILD, slot);
-                u.failed_at = a.u(A::FAILED, slot);
-                a.ldRng(slot, vw.seed, ls, r);
-                const uint32_t fl = a.u(A::FLAGS, slot);
-                st.med = (int)(fl & 255u) - 1;
-                st.depth = (int)(fl >> 8 & 255u);
-                st.mode = (int)(fl >> 16 & 63u);
-                st.walk = (int)(fl >> 22 & 3u);
-                st.walk_surf = (fl >> 24 & 1u) != 0;
-                st.walk_add = (fl >> 25 & 1u) != 0;
-                st.walk_cpdf = a.r(A::CPDF, slot);
-                st.hface = -1;
-                st.ro = a.ldv(A::RO, slot);
-                st.rd = fl & A::RD_CONST ? Dv<N>(a.ld(A::RD, slot)) : a.ldv(A::RD, slot);
-                st.beta = a.lds(A::BETA, slot);
-                alive = true;
-            }
-            Ds<N> L;
-            if (alive) {
-                AdEdgeOut<N> eo{a, slot, false};
-                alive = adBounce<N>(T, P, r, st, L, u, stats, eo);
-                edge = eo.set;
-            }
+            if (adLoad<N>(S, P, B, a, slot, r, st, u))
+                adBounce<N, AdPass::FORWARD>(T, P, a, slot, r, st, u, stats, nullptr, alive, edge);
             nlk += r.nlk;
             a.u(A::CHILD, slot) = u.child;
             a.u(A::FAILED, slot) = u.failed_at;
             if (alive || edge) a.stRng(slot, r);
-            if (alive) {
-                const bool rdc = st.rd.gradZero(0._r);
-                a.u(A::FLAGS, slot) = (uint32_t)(st.med + 1) | (uint32_t)st.depth << 8 | (uint32_t)st.mode << 16 |
-                                      (uint32_t)st.walk << 22 | (st.walk_surf ? 1u << 24 : 0u) | (st.walk_add ? 1u << 25 : 0u) |
-                                      (rdc ? A::RD_CONST : 0u);
-                a.r(A::CPDF, slot) = st.walk_cpdf;
-                if (rdc) a.st(A::RD, slot, st.rd.val());
-                else a.stv(A::RD, slot, st.rd);
-                a.sts(A::BETA, slot, st.beta);
-            }
-            if (alive && !edge) a.stv(A::RO, slot, st.ro);   // an edge term has stored its vertex, the next ray's origin
-            if (first) a.sts(A::L, slot, L);
-            else a.sts(A::L, slot, a.lds(A::L, slot) + L);
         }
-        appendSlots(alive, slot, B.out, B.cnt + 4);
-        appendSlots(edge, slot, B.edges, B.cnt + 2);
+        appendSlots(alive, slot, B.out, B.cnt + 4 * AD_CNT);
+        appendSlots(edge, slot, B.edges, B.cnt + 2 * AD_CNT);
+    }
+    flushWork(work, 0, T.nbox, T.ntri, nlk, T.nseg);
+}
+
+// Path-replay adjoint of the density derivative of the interior terms: the host restricts the
+// terms to emission, surface and volume interior (no edge or Lins sub-paths), so nothing is
+// pushed. Pass 0 lists the samples whose pixel has a loss gradient (dimg, into EBETA as
+// gradient / spp), pass 1 those of them that have radiance (L, into ETHR).
+template <int N> __global__ __launch_bounds__(256) void k_adj_list(DScene S, AdBatch B, const float *dimg, int pass) {
+    using A = AdSlots<N>;
+    const A a = slotsOf<N>(B);
+    const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
+    bool put = false;
+    if (slot < B.m) {
+        if (pass == 0) {
+            const uint64_t sid = B.s0 + slot;
+            const DView &vw = S.views[viewOf(S, sid)];
+            const size_t gp = (size_t)vw.pix0 + (size_t)((sid - vw.s0) / (uint64_t)vw.spp);   // pixel of the concatenated gradient images
+            const f3 adj = ld3(dimg + 3 * gp) * (1.0_r / vw.spp);
+            put = !allZero(adj, 0._r);
+            a.st(A::EBETA, slot, adj);
+        } else if (!allZero(a.ld(A::EBETA, slot), 0._r)) {
+            const f3 Lt = a.ld(A::L, slot);
+            put = !allZero(Lt, 0._r);
+            a.st(A::ETHR, slot, Lt);
+        }
+    }
+    // one append per block: waves' appends to one counter take about 11 ns each
+    __shared__ uint32_t len[4], base;
+    const uint64_t m = __ballot(put);
+    if ((threadIdx.x & 63) == 0) len[threadIdx.x / 64] = (uint32_t)__popcll(m);
+    __syncthreads();
+    if (threadIdx.x == 0) base = atomicAdd(B.cnt, len[0] + len[1] + len[2] + len[3]);
+    __syncthreads();
+    if (put) {
+        uint32_t at = base + (uint32_t)__popcll(m & __lanemask_lt());
+        for (unsigned k = 0; k < threadIdx.x / 64; ++k) at += len[k];
+        B.out[at] = slot;
+    }
+}
+// One bounce of the replay: like k_ad_bounce, adding d loss / d node density of medium pmed's
+// grid into grad.
+template <int N>
+__global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_adj_bounce(DScene S, RenderParams P, AdBatch B, double *grad,
+                                                                              int pmed, unsigned *stats,
+                                                                              unsigned long long *work) {
+    using A = AdSlots<N>;
+    const A a = slotsOf<N>(B);
+    ListShare share(B.cnt + AD_CNT, B.cnt[0]);
+    if (share.idleBlock()) return;
+    Tracer<N> T(S);
+    T.useLdsTree(P);
+    uint32_t nlk = 0;
+    for (; share.more(); share.next()) {
+        uint32_t li, slot = 0;
+        bool alive = false, edge = false;
+        if (share.item(li)) {
+            slot = B.in[li];
+            AdState<N> st;
+            Rng r;
+            Pusher u{nullptr, nullptr, 0, 0, 0, 0, 0, Pusher::NO_FAIL};
+            const AdjCtx ac{grad, S.media + pmed, a.ld(A::EBETA, slot), a.ld(A::ETHR, slot)};
+            if (adLoad<N>(S, P, B, a, slot, r, st, u))
+                adBounce<N, AdPass::SCATTER>(T, P, a, slot, r, st, u, stats, &ac, alive, edge);
+            nlk += r.nlk;
+            if (alive) a.stRng(slot, r);
+        }
+        appendSlots(alive, slot, B.out, B.cnt + 4 * AD_CNT);
     }
     flushWork(work, 0, T.nbox, T.ntri, nlk, T.nseg);
 }
@@ -245,7 +506,7 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_EDGE_WAVES) void k_ad_edges(DSce
                                                                           unsigned long long *work) {
     using A = AdSlots<N>;
     const A a = slotsOf<N>(B);
-    ListShare share(B.cnt + 3, B.cnt[2]);
+    ListShare share(B.cnt + 3 * AD_CNT, B.cnt[2 * AD_CNT]);
     if (share.idleBlock()) return;
     Tracer<N> T(S);
     T.useLdsTree(P);

@@ -27,12 +27,15 @@ hipError_t launch_finalize(const DScene &S, const RenderParams &P, int npix, int
                            const void *acc_pe, float *out, unsigned *st, hipStream_t sm) {
     return DT_BY_PREC(S, launch_finalize, S, P, npix, pix0, spp, has_pe, acc, acc_pe, out, st, sm);
 }
-hipError_t launch_adjoint(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg, float *grad,
+hipError_t launch_adjoint(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg, double *grad,
                           int pmed, unsigned *st, unsigned long long *work, hipStream_t sm) {
     return DT_BY_PREC(S, launch_adjoint, S, P, s0, n, dimg, grad, pmed, st, work, sm);
 }
 hipError_t launch_fill32(void *p, uint64_t n, uint32_t v, hipStream_t sm) { return p32::launch_fill32(p, n, v, sm); }
 hipError_t launch_add_u32(unsigned *dst, const unsigned *src, hipStream_t sm) { return p32::launch_add_u32(dst, src, sm); }
+hipError_t launch_add_sums(float *dst, const double *src, uint64_t n, hipStream_t sm) {
+    return p32::launch_add_sums(dst, src, n, sm);
+}
 hipError_t launch_load_density(float *dst, const float *src, uint64_t n, unsigned *maxbits, hipStream_t sm) {
     return p32::launch_load_density(dst, src, n, maxbits, sm);
 }

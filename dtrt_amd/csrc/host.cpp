@@ -682,8 +682,9 @@ struct Scene : Obj {
         for (void *p : pe_bufs) (void)hipFree(p);
         for (auto *b : {&edgebuf, &ecdfbuf, &lightbuf, &refitbuf, &shapecdfbuf}) if (b->p) (void)hipFree(b->p);
         for (auto &b : bufs) if (b.p) (void)hipFree(b.p);
-        for (auto *b : {&acc, &acc_pe, &queue, &qcount, &stats, &work, &outbuf, &ovf[0], &ovf[1], &viewbuf, &tunebuf, &adstate})
+        for (auto *b : {&acc, &acc_pe, &queue, &qcount, &stats, &work, &outbuf, &ovf[0], &ovf[1], &viewbuf, &tunebuf, &adstate.b, &adjstate.b})
             if (b->p) (void)hipFree(b->p);
+        for (auto &b : gradsum) if (b.p) (void)hipFree(b.p);
         for (auto &e : ev) if (e) (void)hipEventDestroy(e);
         if (caller_ev) (void)hipEventDestroy(caller_ev);
         if (stream) (void)hipStreamDestroy(stream);
@@ -697,7 +698,10 @@ struct Scene : Obj {
     std::vector<Medium *> media;
     DScene S;
     std::vector<DevBuf> bufs;
-    DevBuf acc, acc_pe, queue, qcount, stats, work, outbuf, ovf[2], viewbuf, adstate;
+    DevBuf acc, acc_pe, queue, qcount, stats, work, outbuf, ovf[2], viewbuf;
+    struct AdBuf { DevBuf b; unsigned slots = 0, tried = 0; };   // slots: the samples that b holds
+    AdBuf adstate, adjstate;        // path state of the staged AD kernels: the renders', the adjoint's
+    std::vector<DevBuf> gradsum;    // per medium: its density gradient's sums, a double per node
     std::vector<DMedium> hmed;   // host copy of the device media records
     struct PECache { int npe = 0; double pe_sum = 0; const double *cdf = nullptr; const float *pe = nullptr; };
     std::vector<void *> pe_bufs;   // device buffers of the primary-edge cache (freed when geometry changes)
@@ -752,18 +756,27 @@ struct Scene : Obj {
     // 262 -> 220 ms in float, against 64.
     int tune_ad_block = 64, tune_child_block = 256;
     DevBuf tunebuf;
-    unsigned ad_slots = 0;   // samples that adstate holds
-    // The path state of the staged AD kernels for chunks of up to `chunk` samples.
-    bool useAdState(RenderParams &P, uint64_t chunk) {
-        const unsigned want = (unsigned)std::min<uint64_t>(AD_SLOTS, (chunk + 63) / 64 * 64);
-        if (ad_slots < want) {
-            if (!ensure(adstate, adStateBytes(nder, S.f64 != 0, want))) return false;
-            ad_slots = want;
+    // The path state of the staged AD kernels for chunks of up to `chunk` samples of `lanes`
+    // lanes, or for fewer at once: where memory is short, and where a larger one would take
+    // the buffers away from a captured graph that can be replayed.
+    bool useAdState(RenderParams &P, uint64_t chunk, int lanes, AdBuf &a) {
+        unsigned want = (unsigned)std::min<uint64_t>(AD_SLOTS, (chunk + 63) / 64 * 64);
+        if (a.tried < want && !(a.slots && replayable())) {
+            a.tried = want;
+            a.slots = 0;
+            while (!ensure(a.b, adStateBytes(lanes, S.f64 != 0, want))) {
+                (void)hipGetLastError();
+                if (want <= 1u << 16) { a.tried = 0; return false; }
+                want = want / 2 / 64 * 64;
+            }
+            a.slots = want;
         }
-        P.ad_state = static_cast<char *>(adstate.p);
-        P.ad_slots = ad_slots;
+        P.ad_state = static_cast<char *>(a.b.p);
+        P.ad_slots = a.slots;
         return true;
     }
+    // The adjoint's kernels run at one lane (launch_adjoint).
+    bool useAdjState(RenderParams &P, uint64_t chunk) { return useAdState(P, chunk, 1, adjstate); }
 
     template <class T> const T *upload(const std::vector<T> &v) {
         if (v.empty()) return nullptr;
@@ -807,7 +820,17 @@ struct Scene : Obj {
     bool captureViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, float *const *images);
     int replayViews(const uint64_t *seeds);
     std::vector<void *> graphBuffers() const {
-        return {viewbuf.p, acc.p, acc_pe.p, queue.p, qcount.p, stats.p, work.p, ovf[0].p, ovf[1].p, adstate.p};
+        return {viewbuf.p, acc.p, acc_pe.p, queue.p, qcount.p, stats.p, work.p, ovf[0].p, ovf[1].p, adstate.b.p};
+    }
+    std::vector<void *> stepBuffers(int med) const {
+        std::vector<void *> b = graphBuffers();
+        b.push_back(stepbuf.p);
+        b.push_back(adjstate.b.p);
+        b.push_back(med < (int)gradsum.size() ? gradsum[med].p : nullptr);
+        return b;
+    }
+    bool replayable() const {
+        return (graph.x && graph.bufs == graphBuffers()) || (stepg.x && stepg.bufs == stepBuffers(stepg.args.med));
     }
     bool setupViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, std::vector<DView> &hv,
                     std::vector<uint64_t> &pe_total, Bump *pool = nullptr);
@@ -1451,11 +1474,11 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
     } else {
         cap = std::max<uint64_t>(128, std::min<uint64_t>(queue_budget / P.rec_stride, 0xFFFFFFF0ull));
         max_chunk = std::min<uint64_t>(tune_max_chunk, std::max<uint64_t>(total, 64));
-        if (ad_kind == AD_VOLPATH && !useAdState(P, max_chunk)) return false;
         if (!ensure(acc, img * es) || !ensure(acc_pe, (size_t)nder * npix * 3 * es) || !ensure(qcount, 64) ||
             !ensure(stats, 64 * 4) || !ensure(work, 16 * 8) || !ensure(queue, (size_t)cap * P.rec_stride) ||
             !ensure(ovf[0], (size_t)max_chunk * 16) || !ensure(ovf[1], (size_t)max_chunk * 16))
             return false;
+        if (ad_kind == AD_VOLPATH && !useAdState(P, max_chunk, nder, adstate)) return false;
         A = acc.p;
         APE = acc_pe.p;
         Q = static_cast<char *>(queue.p);
@@ -1611,8 +1634,8 @@ bool Scene::captureViews(int nv, const Camera *const *cams, const dtrt_render_op
     const uint64_t cap = std::max<uint64_t>(128, std::min<uint64_t>(queue_budget / P.rec_stride, 0xFFFFFFF0ull));
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
-    P.ad_state = static_cast<char *>(adstate.p);
-    P.ad_slots = ad_slots;
+    P.ad_state = static_cast<char *>(adstate.b.p);
+    P.ad_slots = adstate.slots;
     int dev = 0, ncu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1803,8 +1826,8 @@ bool Scene::captureStep(StepArgs &a) {
     const uint64_t cap = std::max<uint64_t>(128, std::min<uint64_t>(queue_budget / P.rec_stride, 0xFFFFFFF0ull));
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
-    P.ad_state = static_cast<char *>(adstate.p);
-    P.ad_slots = ad_slots;
+    P.ad_state = static_cast<char *>(adstate.b.p);
+    P.ad_slots = adstate.slots;
     int dev = 0, ncu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1817,6 +1840,7 @@ bool Scene::captureStep(StepArgs &a) {
     uint4 *OV = static_cast<uint4 *>(ovf[0].p);
     const DMedium &m = hmed[a.med];
     const uint64_t ngrid = (uint64_t)m.res[0] * m.res[1] * m.res[2];
+    double *dsum = static_cast<double *>(gradsum[a.med].p);
     const uint64_t achunk = uint64_t(1) << 22;
     HIPCHK(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     auto issue = [&]() -> hipError_t {
@@ -1852,8 +1876,10 @@ bool Scene::captureStep(StepArgs &a) {
             if (a.pgrad) GCHK(launch_contract(a.images[v], dimg + (size_t)hvf[v].pix0 * 3, n, nder, a.pgrad, stream));
         }
         GCHK(launch_fill32(a.dgrid, ngrid, 0u, stream));
+        GCHK(launch_fill32(dsum, 2 * ngrid, 0u, stream));
         for (uint64_t a0 = 0; a0 < atotal; a0 += achunk)
-            GCHK(launch_adjoint(Sa, PA, a0, std::min(achunk, atotal - a0), dimg, a.dgrid, a.med, st + 32, wk, stream));
+            GCHK(launch_adjoint(Sa, PA, a0, std::min(achunk, atotal - a0), dimg, dsum, a.med, st + 32, wk, stream));
+        GCHK(launch_add_sums(a.dgrid, dsum, ngrid, stream));
 #undef GCHK
         return hipSuccess;
     };
@@ -1869,8 +1895,7 @@ bool Scene::captureStep(StepArgs &a) {
     stepg.args = a;
     stepg.hvf = hvf;
     stepg.hva = hva;
-    stepg.bufs = graphBuffers();
-    stepg.bufs.push_back(stepbuf.p);
+    stepg.bufs = stepBuffers(a.med);
     return true;
 }
 
@@ -1879,9 +1904,7 @@ bool Scene::captureStep(StepArgs &a) {
 // and the step ran eagerly instead (exact either way), -1 on error.
 int Scene::replayStep(const uint64_t *seeds) {
     if (!stepg.x) { g_err = "replay_step: no captured step"; return -1; }
-    std::vector<void *> now = graphBuffers();
-    now.push_back(stepbuf.p);
-    if (now != stepg.bufs) { g_err = "replay_step: an eager render reallocated the buffers; capture again"; return -1; }
+    if (stepBuffers(stepg.args.med) != stepg.bufs) { g_err = "replay_step: an eager render reallocated the buffers; capture again"; return -1; }
     if (!afterCaller()) return -1;
     const int nv = (int)stepg.hvf.size();
     for (int v = 0; v < nv; ++v) {
@@ -1987,6 +2010,10 @@ bool Scene::renderAdjointViews(int nv, const Camera *const *cams, const dtrt_ren
     uint64_t total = 0;
     P.npix = 0;
     for (int v = 0; v < nv; ++v) { P.npix += hv[v].npix; total += (uint64_t)hv[v].npix * hv[v].spp; }
+    const uint64_t ngrid = (uint64_t)hmed[med].res[0] * hmed[med].res[1] * hmed[med].res[2];
+    gradsum.resize(hmed.size());
+    if (!useAdjState(P, std::min<uint64_t>(total, AD_SLOTS)) || !ensure(gradsum[med], ngrid * 8)) return false;
+    double *sum = static_cast<double *>(gradsum[med].p);
     if (Pout) *Pout = P;
     if (total_out) *total_out = total;
     if (!launch) return true;
@@ -2002,8 +2029,10 @@ bool Scene::renderAdjointViews(int nv, const Camera *const *cams, const dtrt_ren
     std::memset(kernel_ms, 0, sizeof(kernel_ms));
     std::memset(kernel_launches, 0, sizeof(kernel_launches));
     HIPCHK(hipEventRecord(ev[0], stream));
+    HIPCHK(launch_fill32(sum, 2 * ngrid, 0u, stream));
     for (uint64_t s0 = 0; s0 < total; s0 += chunk)
-        HIPCHK(launch_adjoint(S, P, s0, std::min(chunk, total - s0), dimg, grad, med, st, wk, stream));
+        HIPCHK(launch_adjoint(S, P, s0, std::min(chunk, total - s0), dimg, sum, med, st, wk, stream));
+    HIPCHK(launch_add_sums(grad, sum, ngrid, stream));
     HIPCHK(hipEventRecord(ev[1], stream));
     HIPCHK(hipEventSynchronize(ev[1]));
     float ms = 0;

@@ -31,9 +31,10 @@ struct RenderParams {
 constexpr int AD_SLOT_WORDS = 15;
 constexpr int adSlotReals(int nder) { return 12 * (nder + 1) + 16; }
 constexpr int AD_MAX_BOUNCES = 200;
+constexpr int AD_CNT = 32;   // words from one counter to the next: a cache line each, since all waves count in them
 constexpr uint64_t adSlotBytes(int nder, bool f64) { return (uint64_t)adSlotReals(nder) * (f64 ? 8 : 4) + AD_SLOT_WORDS * 4 + 12; }
 constexpr uint64_t adStateBytes(int nder, bool f64, uint64_t slots) {
-    return slots * adSlotBytes(nder, f64) + 16 * (AD_MAX_BOUNCES + 3);
+    return slots * adSlotBytes(nder, f64) + 16 * AD_CNT * (AD_MAX_BOUNCES + 3);
 }
 
 // Counters written by the kernels (warnings the reference prints, as counts).
@@ -78,7 +79,7 @@ struct KernelInfo {
 // launch_adjoint: path-replay adjoint over AD samples s0 .. s0+n-1 (interior terms only):
 // adds d loss / d node density of medium pmed's grid into grad, given d loss / d pixel.
 // launch_fill32: p[0..n) = v (32-bit words); launch_add_u32: *dst += *src. Kernels, so
-// that captured graphs hold no memset nodes.
+// that captured graphs hold no memset nodes. launch_add_sums: dst += src over n elements.
 // launch_load_density: dst = max(src, 0) over n floats; atomicMax of the result's bits
 // into *maxbits.
 // launch_l2_grad: one view of the L2 loss sum (I - T)^2: dimg = 2 (I - T) over n floats,
@@ -105,9 +106,10 @@ struct KernelInfo {
     hipError_t launch_finalize(const DScene &S, const RenderParams &P, int npix, int pix0, int spp, int has_pe,          \
                                const void *acc, const void *acc_pe, float *out, unsigned *st, hipStream_t sm);           \
     hipError_t launch_adjoint(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg,        \
-                              float *grad, int pmed, unsigned *st, unsigned long long *work, hipStream_t sm);            \
+                              double *grad, int pmed, unsigned *st, unsigned long long *work, hipStream_t sm);           \
     hipError_t launch_fill32(void *p, uint64_t n, uint32_t v, hipStream_t sm);                                           \
     hipError_t launch_add_u32(unsigned *dst, const unsigned *src, hipStream_t sm);                                       \
+    hipError_t launch_add_sums(float *dst, const double *src, uint64_t n, hipStream_t sm);                               \
     hipError_t launch_load_density(float *dst, const float *src, uint64_t n, unsigned *maxbits, hipStream_t sm);         \
     hipError_t launch_l2_grad(const float *img, const float *target, float *dimg, uint64_t n, double *loss,             \
                               hipStream_t sm);                                                                           \

@@ -155,30 +155,26 @@ template <int N> struct Tracer {
             if (f < 0) return Ds<N>();
             if (inter == 0) first_face = f;
             if (first_only) return Ds<N>();
-            // At N >= 8 a null crossing takes the distance alone and the full hit record
-            // is refined only at a light (the same t, recomputed): fewer dual operations
-            // per crossing where each carries many tangents. Measured: dielectric scene
-            // at N = 8 8% faster, the N = 3 benchmark scene 5% slower (kept there as is).
-            HitAD<N> nh;
-            Df<N> tmax;
+            // a null crossing takes the distance alone; at a light, the rest of the hit is
+            // needed without tangents (the same record), unless its emission depends on
+            // the shading normal
             f3 gnv;
-            if constexpr (N >= 8) {
-                tmax = hitDistanceAD<N>(S, f, o, d, gnv);
-            } else {
-                refineHitAD<N>(S, f, o, d, nh);
-                tmax = nh.t;
-                gnv = nh.gn.val();
-            }
+            const Df<N> tmax = hitDistanceAD<N>(S, f, o, d, gnv);
             const DShape &sh = shapeOf(S, f);
             dist += tmax;
             if (med >= 0) T *= mediumTransmittanceAD<N>(S.media[med], o, d, tmin, tmax, r, scx);
             if (sh.light_id >= 0) {
-                if constexpr (N >= 8) refineHitAD<N>(S, f, o, d, nh);
-                f3 dd = nh.p.val() - scat;
-                real G = nh.wi.z.v / dot(dd, dd);
+                Hit nh;
+                refineHit(S, f, o.val(), dv, nh);
+                f3 dd = nh.p - scat;
+                real G = nh.wi.z / dot(dd, dd);
                 pdf_nee = S.light_pmf[sh.light_id] / (S.light_areas[sh.light_id] * G);
                 if (far_face) { *far_face = f; *far_t = dist.v; }
-                return emitterEvalAD<N>(S.emitters[sh.light_id], nh, -d) * T;
+                const DEmitter &e = S.emitters[sh.light_id];
+                if (e.type == EMIT_AREA) return Ds<N>(emitterEval(e, nh.gn, nh.sn, -dv)) * T;
+                HitAD<N> ah;
+                refineHitAD<N>(S, f, o, d, ah);
+                return emitterEvalAD<N>(e, ah, -d) * T;
             }
             if (inter == max_inter || bsdfOf(S, sh).type != BSDF_NULL) return Ds<N>();
             if (isTransition(sh)) med = targetMedium(sh, gnv, dv);
