@@ -46,8 +46,12 @@ struct fv3 {
     float x, y, z;
 };
 DI fv3 fsub(fv3 a, fv3 b) { return {a.x - b.x, a.y - b.y, a.z - b.z}; }
-DI float fdot(fv3 a, fv3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-DI fv3 fcross(fv3 a, fv3 b) { return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
+// Which products are fused is written out here and in traceClosest: which triangle a ray
+// near an edge hits depends on it, and the compiler's own choice changes with the code around.
+DI float fdot(fv3 a, fv3 b) { return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y)); }
+DI fv3 fcross(fv3 a, fv3 b) {
+    return {__builtin_fmaf(a.y, b.z, -(a.z * b.y)), __builtin_fmaf(a.z, b.x, -(a.x * b.z)), __builtin_fmaf(a.x, b.y, -(a.y * b.x))};
+}
 
 // Closest hit in [tnear, tfar] of the fp32-rounded ray: global face id (or -1), its
 // t, and the box and triangle tests done. Inlined at every call site: as an
@@ -83,6 +87,7 @@ HDI size_t ldsNodesBytes(int lds_nodes) { return ((size_t)lds_nodes * LDS_NODE *
 // Only kernels built with treePrefixInLds<N>() read a part of the nodes from LDS: their
 // traversal tests each node's index against lds_nodes, which the others save by
 // reading LDS only when the whole tree is there (lds_tris), a launch-uniform test.
+// A kernel with a variant for each place (Tree, below) reads a prefix in its HBM variant.
 // Measured back to back on one GPU: the N = 3 benchmark scene (whole tree in LDS) renders in 0.652 s
 // with the uniform test and 0.670 s with the per-node one; the 100K-face dielectric
 // scene at N = 8 in 7.02 s without and 6.84 s with a prefix of its tree in LDS.
@@ -127,7 +132,15 @@ DI Hit2 boxesHit(fv3 o, fv3 inv, float2 nx, float2 ny, float2 nz, float2 fx, flo
     return {tl <= ul, tr <= ur};
 }
 
-template <bool PREFIX = false>
+// Where the tree of a kernel's launches is: either place, read by a launch-uniform test (ANY),
+// wholly in LDS (LDS), or in HBM but for a prefix of its nodes (HBM). A node from HBM costs a
+// wave about twice one from LDS however few lanes wait for it (1,350 against 700 cycles), and
+// a step of the 50K-face dielectric scene's children had 5.6 lanes: with the tree in HBM the
+// wave goes over to its leaves as soon as fewer than half of its lanes are at inner nodes
+// (that scene's child kernel at 8 lanes 41.5 -> 36.7 ms). In LDS the votes cost more than the
+// lanes they win (benchmark children 193 -> 220 ms).
+enum class Tree { ANY, LDS, HBM };
+template <bool PREFIX = false, Tree WHERE = Tree::ANY>
 DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3 o_, f3 d_, real tnear_, real tfar_,
                          int lds_nodes = 0, bool lds_tris = false, int stack_depth = DTRT_BVH_STACK) {
     const fv3 o{(float)o_.x, (float)o_.y, (float)o_.z}, d{(float)d_.x, (float)d_.y, (float)d_.z};
@@ -151,11 +164,18 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
     while (node != DONE) {
         // inner nodes until this lane reaches a leaf or runs out of nodes; the wave then
         // tests the leaves it reached together
-        while (node >= 0) {
+        while (true) {
+            if constexpr (WHERE == Tree::HBM) {
+                const uint64_t in = __ballot(node >= 0);
+                if (in == 0 || 2 * __popcll(in) < __popcll(__ballot(node != DONE))) break;
+                if (node < 0) continue;
+            } else {
+                if (node < 0) break;
+            }
             const int popped = *top;   // read with the node, so that a pop waits for nothing more
             float2 nx, ny, nz, fx, fy, fz;
             int cl, cr;
-            if (PREFIX ? node < lds_nodes : lds_tris) {
+            if (WHERE == Tree::LDS || (PREFIX ? node < lds_nodes : WHERE == Tree::ANY && lds_tris)) {
                 const int w = LDS_NODE * node;
                 auto pair = [w](const float *p) { return *reinterpret_cast<const float2 *>(p + w); };
                 nx = pair(lx); ny = pair(ly); nz = pair(lz);
@@ -181,12 +201,13 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
             top = hl && hr ? top + stride : hl || hr ? top : top - stride;
         }
         if (node == DONE) break;
+        if (WHERE == Tree::HBM && node >= 0) continue;
         int enc = ~node;
         int first = enc >> 4, cnt = enc & 15;
         ntri += cnt;
         for (int k = first; k < first + cnt; ++k) {
             float4 v0, e1, e2;
-            if (lds_tris) {
+            if (WHERE == Tree::LDS || (WHERE == Tree::ANY && lds_tris)) {
                 const float4 *tp = reinterpret_cast<const float4 *>(lds + ldsNodesBytes(nnodes) / 4) + 3 * k;
                 v0 = tp[0]; e1 = tp[1]; e2 = tp[2];
             } else {
@@ -202,8 +223,8 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
             float u = fdot(s, pv) * idet;
             if (u < -BEPS || u > 1.0f + BEPS) continue;
             fv3 q = fcross(s, E1);
-            float v = fdot(d, q) * idet;
-            if (v < -BEPS || u + v > 1.0f + BEPS) continue;
+            const float dq = fdot(d, q), v = dq * idet;
+            if (v < -BEPS || __builtin_fmaf(idet, dq, u) > 1.0f + BEPS) continue;   // u + v
             float t = fdot(E2, q) * idet;
             if (t >= tnear && t <= best) { best = t; face = __float_as_int(v0.w); }
         }

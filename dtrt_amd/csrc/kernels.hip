@@ -52,6 +52,10 @@ constexpr int WIDE_BLOCK = 512;
 // Work-group size of the primal path and particle kernels: four waves, so that at their
 // occupancy a small scene's tree fits in LDS beside the traversal stacks (treeLdsFor).
 constexpr int PRIMAL_BLOCK = 256;
+// Primary-edge samples: one group of two waves per SIMD for a CU, so that the tree fits once. 45M
+// samples of the surface scene, with the atomics of 64-thread groups 27.8 ms, in persistent
+// groups of 64 19.1 ms, of 256 11.6 ms, of 512 10.7 ms (13.9 ms with 4 waves per SIMD).
+constexpr int PRIMARY_BLOCK = 512, PRIMARY_WAVES = 2;
 HDI unsigned blockOr64(int b) { return b == 128 || b == 256 ? (unsigned)b : 64u; }
 // Minimum resident waves per SIMD requested from the register allocator (HIP's second
 // __launch_bounds__ argument): bounds the VGPRs of the two path kernels. Per
@@ -62,6 +66,10 @@ HDI unsigned blockOr64(int b) { return b == 128 || b == 256 ? (unsigned)b : 64u;
 #ifndef CHILD_WAVES_F64
 #define CHILD_WAVES_F64 2   // heterogeneous-medium scene, 512^2, 128 spp, nder 3, child kernel per render: 2 waves 413 ms, 4 waves 464 ms (1 wave: 1.5x 2)
 #endif
+// Where the tree lies in HBM a child waits for its nodes one after the other: more waves, at the
+// price of spills. 50K-face dielectric scene, child kernel at 8 lanes 36.7 ms with 2 waves per
+// SIMD, 41.5 with 3, 32.8 with 4, 39.1 with 5; surface scene's tree read from HBM 70.5 -> 62.7 ms.
+#define CHILD_WAVES_HBM 4
 #ifndef AD_WAVES_PER_SIMD
 #define AD_WAVES_PER_SIMD (kF64 ? 1 : 2)   // the surface-only AD kernel and the adjoint
 #endif
@@ -99,14 +107,16 @@ DI int viewOf(const DScene &S, uint64_t sid) {
     return lo;
 }
 
-DI bool writeRecord(const RenderParams &P, char *q, unsigned *qcount, const ChildHdr &h, const real *w, int nw) {
-    unsigned idx = atomicAdd(qcount, 1u);
+DI bool storeRecord(const RenderParams &P, char *q, unsigned idx, const ChildHdr &h, const real *w, int nw) {
     if (idx >= P.qcap) return false;
     char *rec = q + (size_t)idx * P.rec_stride;
     *reinterpret_cast<ChildHdr *>(rec) = h;
     real *wd = reinterpret_cast<real *>(rec + sizeof(ChildHdr));
     for (int i = 0; i < nw; ++i) wd[i] = w[i];
     return true;
+}
+DI bool writeRecord(const RenderParams &P, char *q, unsigned *qcount, const ChildHdr &h, const real *w, int nw) {
+    return storeRecord(P, q, atomicAdd(qcount, 1u), h, w, nw);
 }
 
 // Child pushes of one AD path sample. Children are numbered 1, 2, ... in push order
@@ -556,18 +566,18 @@ __global__ __launch_bounds__(MAX_BLOCK, adWaves<N>()) void k_ad_paths(DScene S, 
 //   PRIMAL_PATH     PathTracer (path.cpp:64-96) and DirectIntegrator (direct.cpp:
 //                   51-85, max depth 1): pathStep, camera ray from tnear ShadowEpsilon.
 // Radiance sums go to acc[pixel][3].
-template <int KIND>
-__global__ __launch_bounds__(PRIMAL_BLOCK, CHILD_WAVES_PER_SIMD) void k_primal_paths(DScene S, RenderParams P, uint64_t s0,
+template <int KIND, Tree WHERE>
+__global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD) void k_primal_paths(DScene S, RenderParams P, uint64_t s0,
                                                                                      uint64_t nsamp, real *acc,
                                                                                      unsigned long long *work) {
     const uint32_t blk = xcdRemap(blockIdx.x, gridDim.x);
-    const uint64_t li = (uint64_t)blk * PRIMAL_BLOCK + threadIdx.x;
+    const uint64_t li = (uint64_t)blk * blockDim.x + threadIdx.x;
     const bool active = li < nsamp;
     const DView &vw = S.views[0];
     const DCamera &cam = vw.cam;
     const uint64_t ls = s0 + li;
     const int pixel = (int)(ls / (uint64_t)vw.spp);
-    Tracer<1> T(S);
+    Tracer<1, WHERE> T(S);
     T.useLdsTree(P);
     Rng r;
     r.init(vw.seed, ls);
@@ -934,12 +944,12 @@ DI int lanesToUse(unsigned n) {
 // Persistent: each lane holds one primal sub-path and advances it one bounce per
 // iteration; a lane whose path has ended takes the next queued record (one atomic
 // per wave on qnext), so the lanes of a wave stay busy until the queue is drained.
-template <int N>
-__global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
+template <int N, Tree WHERE>
+__global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
                                                     unsigned *qnext, real *acc, real *acc_pe, unsigned long long *work) {
     const unsigned n = min(*qcount, P.qcap);
     if (blockIdx.x >= n) return;   // each block before this one has a record
-    Tracer<N> T(S);
+    Tracer<N, WHERE> T(S);
     T.useLdsTree(P);
     const int lane = threadIdx.x & 63;
     const bool use = lane < lanesToUse(n);
@@ -1001,14 +1011,14 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children(D
 
 // Persistent drain of CHILD_PATH records (the surface-only integrators' sub-paths,
 // path.cpp:11-61 from the record's origin and direction), as k_children.
-template <int N>
-__global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_path(DScene S, RenderParams P, const char *q,
+template <int N, Tree WHERE>
+__global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD) void k_children_path(DScene S, RenderParams P, const char *q,
                                                                             const unsigned *qcount, unsigned *qnext,
                                                                             real *acc, real *acc_pe,
                                                                             unsigned long long *work) {
     const unsigned n = min(*qcount, P.qcap);
     if (blockIdx.x >= n) return;   // each block before this one has a record
-    Tracer<N> T(S);
+    Tracer<N, WHERE> T(S);
     T.useLdsTree(P);
     const int lane = threadIdx.x & 63;
     const bool use = lane < lanesToUse(n);
@@ -1053,10 +1063,11 @@ __global__ __launch_bounds__(WIDE_BLOCK, CHILD_WAVES_PER_SIMD) void k_children_p
     flushWork(work, 4, T.nbox, T.ntri, nlk, T.nseg);
 }
 
-// edge_manager.cpp:112-134 + integratorAD.cpp:126-144 for one primary-edge sample
+// edge_manager.cpp:112-134 + integratorAD.cpp:126-144 for one primary-edge sample: whether it
+// has the two records `h` towards dir[0] and dir[1], of weights W and -W.
 template <int N>
-DI void primaryEdgeSample(Tracer<N> &T, const RenderParams &P, const DView &vw, int view, Rng &r, uint64_t sid,
-                          uint64_t total, char *q, unsigned *qcount, unsigned *stats) {
+DI bool primaryEdgeSample(Tracer<N> &T, const RenderParams &P, const DView &vw, int view, Rng &r, uint64_t total, ChildHdr &h,
+                          f3 dir[2], real W[N * 3]) {
     const DCamera &c = vw.cam;
     real u = r.next();
     int idx = sampleReuse(vw.pe_cdf, vw.npe, u, nullptr);   // edge_manager.cpp:112-134
@@ -1072,7 +1083,7 @@ DI void primaryEdgeSample(Tracer<N> &T, const RenderParams &P, const DView &vw, 
         pd[j][1] = g[1] + u * (g[3] - g[1]);
         nz = nz || fabs(pd[j][0]) > EPS || fabs(pd[j][1]) > EPS;
     }
-    if (!nz) return;
+    if (!nz) return false;
     int ipx = (int)floor(px_), ipy = (int)floor(py_);
     double nx = pe[3] - pe[1], ny = pe[0] - pe[2], nl = sqrt(nx * nx + ny * ny);
     nx /= nl;
@@ -1103,19 +1114,17 @@ DI void primaryEdgeSample(Tracer<N> &T, const RenderParams &P, const DView &vw, 
     };
     f3 org{c.c2w[3], c.c2w[7], c.c2w[11]};
     real trans = T.evalTransmittance(org, camdir(px_, py_), false, c.med_id, maxD, r, P.max_bounces - 1);
-    if (!(trans > EPS)) return;
+    if (!(trans > EPS)) return false;
     bool inside = c.cropped ? (ipx >= c.ox && ipx < c.ox + c.cw && ipy >= c.oy && ipy < c.oy + c.ch)
                             : (ipx >= 0 && ipx < c.width && ipy >= 0 && ipy < c.height);
-    if (!inside) return;
+    if (!inside) return false;
     int pix = vw.pix0 + (c.cropped ? (ipx - c.ox) + c.cw * (ipy - c.oy) : ipx + c.width * ipy);
-    real W[N * 3];
     real scale = (real)(vw.pe_sum / (double)total);
 #pragma unroll
     for (int j = 0; j < N; ++j) {
         real w = (real)(nx * pd[j][0] + ny * pd[j][1]) * scale;
         W[3 * j] = w; W[3 * j + 1] = w; W[3 * j + 2] = w;
     }
-    ChildHdr h;
     h.org[0] = org.x; h.org[1] = org.y; h.org[2] = org.z;
     h.pixel = pix;
     h.view = view;
@@ -1125,31 +1134,54 @@ DI void primaryEdgeSample(Tracer<N> &T, const RenderParams &P, const DView &vw, 
     h.face = -1;
     for (int s = 0; s < 2; ++s) {
         double sg = s == 0 ? -1.0 : 1.0;
-        f3 d = camdir(px_ + sg * nx * PRIMARY_DELTA, py_ + sg * ny * PRIMARY_DELTA);
-        h.dir[0] = d.x; h.dir[1] = d.y; h.dir[2] = d.z;
-        uint64_t ck = ((1ull << 62) | sid) * 4 + s;
-        h.key_lo = (uint32_t)ck; h.key_hi = (uint32_t)(ck >> 32);
-        if (s == 1)
-#pragma unroll
-            for (int k = 0; k < N * 3; ++k) W[k] = -W[k];
-        // the queue holds two records per primary-edge sample of the launch: cannot fail
-        if (!writeRecord(P, q, qcount, h, W, N * 3)) atomicAdd(stats + STAT_QUEUE_OVERFLOW, 1u);
+        dir[s] = camdir(px_ + sg * nx * PRIMARY_DELTA, py_ + sg * ny * PRIMARY_DELTA);
     }
+    return true;
 }
 
+// Primary-edge samples s0 .. s0+nsamp-1 of a view, by as many blocks as the device holds: what
+// bounds a sample is not its one ray but the waves' atomics, so a wave keeps its work counters
+// to the end and reserves the records of 64 samples at once.
 template <int N>
-__global__ __launch_bounds__(BLOCK) void k_primary(DScene S, RenderParams P, int view, uint64_t s0, uint64_t nsamp,
-                                                   uint64_t total, char *q, unsigned *qcount, unsigned *stats,
-                                                   unsigned long long *work) {
+__global__ __launch_bounds__(PRIMARY_BLOCK, PRIMARY_WAVES) void k_primary(DScene S, RenderParams P, int view, uint64_t s0, uint64_t nsamp,
+                                                           uint64_t total, char *q, unsigned *qcount, unsigned *stats,
+                                                           unsigned long long *work) {
     Tracer<N> T(S);
     T.useLdsTree(P);
-    const uint64_t li = (uint64_t)blockIdx.x * BLOCK + threadIdx.x;
-    const uint64_t sid = s0 + li;
-    Rng r;
     const DView &vw = S.views[view];
-    r.init(vw.seed, (1ull << 62) | sid);
-    if (li < nsamp) primaryEdgeSample<N>(T, P, vw, view, r, sid, total, q, qcount, stats);
-    flushWork(work, 8, T.nbox, T.ntri, r.nlk, T.nseg);
+    uint32_t nlk = 0;
+    for (uint64_t b = (uint64_t)blockIdx.x * PRIMARY_BLOCK; b < nsamp; b += (uint64_t)gridDim.x * PRIMARY_BLOCK) {
+        const uint64_t li = b + threadIdx.x, sid = s0 + li;
+        ChildHdr h;
+        f3 dir[2];
+        real W[N * 3];
+        bool has = false;
+        if (li < nsamp) {
+            Rng r;
+            r.init(vw.seed, (1ull << 62) | sid);
+            has = primaryEdgeSample<N>(T, P, vw, view, r, total, h, dir, W);
+            nlk += r.nlk;
+        }
+        const uint64_t m = __ballot(has);
+        if (!m) continue;
+        const int lane = threadIdx.x & 63, lead = __ffsll((unsigned long long)m) - 1;
+        unsigned base = 0;
+        if (lane == lead) base = atomicAdd(qcount, 2u * (unsigned)__popcll(m));
+        base = __shfl(base, lead) + 2u * (unsigned)__popcll(m & ((1ull << lane) - 1ull));
+        if (!has) continue;
+        // a sample's two records lie together: their paths start alike, in neighbouring lanes
+        for (int s = 0; s < 2; ++s) {
+            h.dir[0] = dir[s].x; h.dir[1] = dir[s].y; h.dir[2] = dir[s].z;
+            const uint64_t ck = ((1ull << 62) | sid) * 4 + s;
+            h.key_lo = (uint32_t)ck; h.key_hi = (uint32_t)(ck >> 32);
+            if (s == 1)
+#pragma unroll
+                for (int k = 0; k < N * 3; ++k) W[k] = -W[k];
+            // the queue holds two records per primary-edge sample of the launch: cannot fail
+            if (!storeRecord(P, q, base + s, h, W, N * 3)) atomicAdd(stats + STAT_QUEUE_OVERFLOW, 1u);
+        }
+    }
+    flushWork(work, 8, T.nbox, T.ntri, nlk, T.nseg);
 }
 
 // One view: pixels pix0 .. pix0+npix of the accumulators into its image.
@@ -1464,23 +1496,29 @@ template <int N> void WidthOps<N>::launchChildren(const DScene &S, const RenderP
     // launched, since each drains the queue until it is empty
     const unsigned dflt = blockOr64(P.child_block);
     RenderParams Pl = P;
-    auto launch = [&](auto kern) {
-        const unsigned blk = wideGroup(kern, dflt, S, P);
-        const size_t lds = traceLds(blk, S.stack_depth) + treeLdsFor(kern, blk, S, Pl, treePrefixInLds<N>());
+    auto launch = [&](auto in_lds, auto in_hbm) {
+        unsigned blk = wideGroup(in_lds, dflt, S, P);
+        size_t tree = treeLdsFor(in_lds, blk, S, Pl, false);
+        auto kern = in_lds;
+        if (!Pl.lds_tris) {
+            kern = in_hbm;
+            blk = dflt;
+            tree = treeLdsFor(in_hbm, blk, S, Pl, true);
+        }
+        const size_t lds = traceLds(blk, S.stack_depth) + tree;
         const unsigned nb = std::min(std::max(1u, grid * dflt / blk), residentBlocks(kern, blk, lds));
         hipLaunchKernelGGL(kern, dim3(nb), dim3(blk), lds, sm, S, Pl, q, qc, qc + 2, acc, acc_pe, wk);
     };
-    if (P.ad_kind == AD_VOLPATH) launch(k_children<N>);
-    else launch(k_children_path<N>);
+    if (P.ad_kind == AD_VOLPATH) launch(k_children<N, Tree::LDS>, k_children<N, Tree::HBM>);
+    else launch(k_children_path<N, Tree::LDS>, k_children_path<N, Tree::HBM>);
 }
 template <int N> void WidthOps<N>::launchPrimary(const DScene &S, const RenderParams &P, int view, uint64_t s0, uint64_t n,
                                            uint64_t total, char *q, unsigned *qc, unsigned *st, unsigned long long *wk,
                                            hipStream_t sm) {
-    unsigned nb = (unsigned)((n + BLOCK - 1) / BLOCK);
     RenderParams Pl = P;
-    const size_t tl = treeLdsFor(k_primary<N>, BLOCK, S, Pl, treePrefixInLds<N>());
-    hipLaunchKernelGGL(k_primary<N>, dim3(nb), dim3(BLOCK), traceLds(BLOCK, S.stack_depth) + tl, sm, S, Pl, view, s0, n, total, q, qc, st,
-                       wk);
+    const size_t lds = traceLds(PRIMARY_BLOCK, S.stack_depth) + treeLdsFor(k_primary<N>, PRIMARY_BLOCK, S, Pl, treePrefixInLds<N>());
+    const unsigned nb = (unsigned)std::min<uint64_t>((n + PRIMARY_BLOCK - 1) / PRIMARY_BLOCK, residentBlocks(k_primary<N>, PRIMARY_BLOCK, lds));
+    hipLaunchKernelGGL(k_primary<N>, dim3(nb), dim3(PRIMARY_BLOCK), lds, sm, S, Pl, view, s0, n, total, q, qc, st, wk);
 }
 template <int N> void WidthOps<N>::launchFinalize(const RenderParams &P, int npix, int pix0, int spp, int has_pe, const real *acc,
                                             const real *acc_pe, float *out, unsigned *st, hipStream_t sm) {
@@ -1503,9 +1541,11 @@ template <int N> hipError_t WidthOps<N>::kernelInfo(KernelInfo *out, int cap, in
     DT_INFO(k_ad_finish<N>, "k_ad_finish", 256, 0)
     DT_INFO((k_ad_paths<N, AD_PATH>), "k_ad_paths/path", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_ad_paths<N, AD_DIRECT>), "k_ad_paths/direct", MAX_BLOCK, traceLds(MAX_BLOCK))
-    DT_INFO(k_children<N>, "k_children", MAX_BLOCK, traceLds(MAX_BLOCK))
-    DT_INFO(k_children_path<N>, "k_children_path", MAX_BLOCK, traceLds(MAX_BLOCK))
-    DT_INFO(k_primary<N>, "k_primary", BLOCK, traceLds(BLOCK))
+    DT_INFO((k_children<N, Tree::LDS>), "k_children", MAX_BLOCK, traceLds(MAX_BLOCK))
+    DT_INFO((k_children<N, Tree::HBM>), "k_children/hbm", MAX_BLOCK, traceLds(MAX_BLOCK))
+    DT_INFO((k_children_path<N, Tree::LDS>), "k_children_path", MAX_BLOCK, traceLds(MAX_BLOCK))
+    DT_INFO((k_children_path<N, Tree::HBM>), "k_children_path/hbm", MAX_BLOCK, traceLds(MAX_BLOCK))
+    DT_INFO(k_primary<N>, "k_primary", PRIMARY_BLOCK, traceLds(PRIMARY_BLOCK))
     DT_INFO(k_adj_bounce<N>, "k_adj_bounce", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
     DT_INFO(k_adj_list<N>, "k_adj_list", 256, 0)
     DT_INFO(k_grid<N>, "k_grid", BLOCK, 0)
@@ -1620,27 +1660,26 @@ hipError_t launch_trace(const DScene &S, const float *rays, int n, int *face, fl
 }
 hipError_t launch_primal_paths(const DScene &S, const RenderParams &P, int kind, uint64_t s0, uint64_t n, void *acc,
                               unsigned long long *work, hipStream_t sm) {
-    const uint64_t nb = (n + PRIMAL_BLOCK - 1) / PRIMAL_BLOCK;
-    if (nb > 0x7FFFFFFFull) return hipErrorInvalidValue;
+    if ((n + PRIMAL_BLOCK - 1) / PRIMAL_BLOCK > 0x7FFFFFFFull) return hipErrorInvalidValue;
     real *A = static_cast<real *>(acc);
     RenderParams Pl = P;
-    const size_t lds = traceLds(PRIMAL_BLOCK, S.stack_depth);
-    if (kind == PRIMAL_SIMPLE) {
-        const size_t tl = treeLdsFor(k_primal_paths<PRIMAL_SIMPLE>, PRIMAL_BLOCK, S, Pl, false);
-        hipLaunchKernelGGL(k_primal_paths<PRIMAL_SIMPLE>, dim3((unsigned)nb), dim3(PRIMAL_BLOCK), lds + tl, sm, S, Pl, s0,
-                           n, A, work);
-    } else if (kind == PRIMAL_PATH) {
-        const size_t tl = treeLdsFor(k_primal_paths<PRIMAL_PATH>, PRIMAL_BLOCK, S, Pl, false);
-        hipLaunchKernelGGL(k_primal_paths<PRIMAL_PATH>, dim3((unsigned)nb), dim3(PRIMAL_BLOCK), lds + tl, sm, S, Pl, s0, n,
+    auto launch = [&](auto in_lds, auto in_hbm) {
+        unsigned blk = wideGroup(in_lds, PRIMAL_BLOCK, S, P);
+        size_t tree = treeLdsFor(in_lds, blk, S, Pl, false);
+        auto kern = in_lds;
+        if (!Pl.lds_tris) {
+            kern = in_hbm;
+            blk = PRIMAL_BLOCK;
+            tree = treeLdsFor(in_hbm, blk, S, Pl, true);
+        }
+        hipLaunchKernelGGL(kern, dim3((unsigned)((n + blk - 1) / blk)), dim3(blk), traceLds(blk, S.stack_depth) + tree, sm, S, Pl, s0, n,
                            A, work);
-    } else if (kind == PRIMAL_VOLPATH) {
-        const size_t tl = treeLdsFor(k_primal_paths<PRIMAL_VOLPATH>, PRIMAL_BLOCK, S, Pl, false);
-        hipLaunchKernelGGL(k_primal_paths<PRIMAL_VOLPATH>, dim3((unsigned)nb), dim3(PRIMAL_BLOCK), lds + tl, sm, S, Pl, s0,
-                           n, A, work);
-    } else {
-        return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+        return hipGetLastError();
+    };
+    if (kind == PRIMAL_SIMPLE) return launch(k_primal_paths<PRIMAL_SIMPLE, Tree::LDS>, k_primal_paths<PRIMAL_SIMPLE, Tree::HBM>);
+    if (kind == PRIMAL_PATH) return launch(k_primal_paths<PRIMAL_PATH, Tree::LDS>, k_primal_paths<PRIMAL_PATH, Tree::HBM>);
+    if (kind == PRIMAL_VOLPATH) return launch(k_primal_paths<PRIMAL_VOLPATH, Tree::LDS>, k_primal_paths<PRIMAL_VOLPATH, Tree::HBM>);
+    return hipErrorInvalidValue;
 }
 hipError_t launch_particles(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, void *acc,
                             unsigned long long *work, hipStream_t sm) {
@@ -1682,9 +1721,12 @@ hipError_t kernel_info(const DScene &S, KernelInfo *out, int cap, int *count) {
 #undef DT_INFO_N
         default: return hipErrorInvalidValue;
     }
-    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH>, "k_primal_paths/volpath", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
-    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE>, "k_primal_paths/simple", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
-    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_PATH>, "k_primal_paths/path", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::LDS>, "k_primal_paths/volpath", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::HBM>, "k_primal_paths/volpath/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE, Tree::LDS>, "k_primal_paths/simple", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE, Tree::HBM>, "k_primal_paths/simple/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_PATH, Tree::LDS>, "k_primal_paths/path", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_PATH, Tree::HBM>, "k_primal_paths/path/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_particles, "k_particles", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_refit, "k_refit", 256, 0, out, cap, count);
     return e;

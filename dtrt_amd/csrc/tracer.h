@@ -27,7 +27,8 @@ struct LiPath {
     real cpdf;
 };
 
-template <int N> struct Tracer {
+template <int N, Tree WHERE = Tree::ANY> struct Tracer {
+    static constexpr bool PREFIX = WHERE == Tree::HBM || (WHERE == Tree::ANY && treePrefixInLds<N>());
     const DScene &S;
     uint32_t nbox = 0, ntri = 0, nseg = 0;   // work counters: box tests, triangle tests, traced segments
     int lds_nodes = 0;                       // nodes [0, lds_nodes) are in LDS (treeToLds)
@@ -36,13 +37,13 @@ template <int N> struct Tracer {
     // At the top of a kernel, by every thread: copy what the launch made room for into
     // LDS (a kernel that reads no prefix is given the whole tree or nothing).
     DI void useLdsTree(const RenderParams &P) {
-        if constexpr (treePrefixInLds<N>()) {
+        if constexpr (PREFIX) {
             if (P.lds_nodes > 0) {
                 treeToLds(S, P.lds_nodes, P.lds_tris != 0);
                 lds_nodes = P.lds_nodes;
                 lds_tris = P.lds_tris != 0;
             }
-        } else if (P.lds_tris) {
+        } else if (WHERE == Tree::LDS || P.lds_tris) {
             treeToLds(S, S.nnodes, true);
             lds_tris = true;
         }
@@ -50,7 +51,7 @@ template <int N> struct Tracer {
 
     DI int trace(f3 o, f3 d, real tnear, real tfar, real &t) {
         nseg++;
-        TraceHit h = traceClosest<treePrefixInLds<N>()>(S.nodes, S.tris, S.nnodes, o, d, tnear, tfar, lds_nodes, lds_tris,
+        TraceHit h = traceClosest<PREFIX, WHERE>(S.nodes, S.tris, S.nnodes, o, d, tnear, tfar, lds_nodes, lds_tris,
                                                         S.stack_depth);
         nbox += h.nbox;
         ntri += h.ntri;

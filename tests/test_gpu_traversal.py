@@ -90,3 +90,20 @@ def test_middle_trees_render_the_same_from_lds_and_hbm(gpu, subdiv, rtol):
     for lane in range(4):
         assert np.abs(lds[lane]).max() > 0
         assert np.allclose(lds[lane], hbm[lane], rtol=rtol, atol=rtol * 1e-2 * np.abs(lds[lane]).max()), lane
+
+
+@pytest.mark.parametrize("subdiv", [2, 3, 4])
+@pytest.mark.parametrize("kind", [1, 2, 3])
+def test_primal_images_do_not_depend_on_where_the_tree_is(gpu, subdiv, kind):
+    """320, 1,280 and 5,120 triangles: wholly in LDS for work-groups of four waves, of eight, and
+    a prefix of the nodes only; against the tree in HBM alone. The same paths, each pixel's
+    sum in another order (doubles rounded to float: 1e-6)."""
+    d = scenes.ico_surface(nder=1, res=37, spp=5)
+    v, f = scenes.icosphere(subdiv, 0.5, (0, 0.5, 0))
+    d.shapes[1] = scenes.ShapeDesc(v, f, bsdf_id=1, velocities=np.zeros((1, len(v), 3), np.float32))
+    sc = scenes.instantiate(gpu, d)
+    a = scenes.render_primal(gpu, d, seed=9, scene=sc, kind=kind)
+    gpu.set_tree_in_hbm(sc, True)
+    b = scenes.render_primal(gpu, d, seed=9, scene=sc, kind=kind)
+    assert a.max() > 0
+    assert np.allclose(a, b, rtol=1e-6, atol=1e-9)
