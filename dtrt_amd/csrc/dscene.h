@@ -135,7 +135,7 @@ DI Hit2 boxesHit(fv3 o, fv3 inv, float2 nx, float2 ny, float2 nz, float2 fx, flo
 // Where the tree of a kernel's launches is: either place, read by a launch-uniform test (ANY),
 // wholly in LDS (LDS), or in HBM but for a prefix of its nodes (HBM). A node from HBM costs a
 // wave about twice one from LDS however few lanes wait for it (1,350 against 700 cycles), and
-// a step of the 50K-face dielectric scene's children had 5.6 lanes: with the tree in HBM the
+// a step of the 100K-face dielectric scene's children had 5.6 lanes: with the tree in HBM the
 // wave goes over to its leaves as soon as fewer than half of its lanes are at inner nodes
 // (that scene's child kernel at 8 lanes 41.5 -> 36.7 ms). In LDS the votes cost more than the
 // lanes they win (benchmark children 193 -> 220 ms).

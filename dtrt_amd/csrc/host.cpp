@@ -924,7 +924,7 @@ bool frameRotationReady() {
 // spills, private arrays) lives in per-lane scratch that the runtime provisions for every
 // wave the device holds at once. The limits are the largest figures that a kernel has
 // passed the GPU parity suite with, rounded up: 10,360 bytes per lane and 679 MB over the
-// device (a build of the double-precision nder-16 refill kernel: 10,360 B x 64 lanes x 4
+// device (an earlier build of the double-precision nder-16 AD kernel: 10,360 B x 64 lanes x 4
 // waves per CU x 256 CUs; the current build needs 7,104 B). A width-16 build of the
 // single-precision AD-path kernel held to two waves per SIMD, whose spills needed 7.9 KB
 // per lane (1.04 GB over the device), rendered empty images: every path ended after two
@@ -1440,7 +1440,7 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
     const size_t npix = P.npix, img = (size_t)(nder + 1) * npix * 3;
     // One queue of child records for both passes. AD samples are launched in chunks
     // sized from the children-per-sample rate seen so far; a sample whose pushes
-    // overflow is replayed exactly (see k_ad_paths). A primary-edge sample pushes at
+    // overflow is replayed exactly (see Pusher). A primary-edge sample pushes at
     // most 2 records, so its chunks never overflow.
     const size_t es = accBytes();
     void *A = nullptr, *APE = nullptr;

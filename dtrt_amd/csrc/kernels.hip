@@ -6,6 +6,8 @@
 //                   paths still alive. They sum the interior terms and push every primal
 //                   sub-path the boundary terms need (2 per accepted edge sample, 1 per
 //                   Lins sample) into an HBM queue.
+//  k_adj_list<N>, k_adj_bounce<N> (ad_stages.h)
+//                   the density adjoint's replay of those paths.
 //  k_ad_paths<N>    the same for the surface-only integrators, one thread per sample.
 //  k_children<N>    one thread per queued sub-path: primal Li / Lins estimate, scattered
 //                   with its per-lane weights into the derivative accumulators.
@@ -64,14 +66,14 @@ HDI unsigned blockOr64(int b) { return b == 128 || b == 256 ? (unsigned)b : 64u;
 #define CHILD_WAVES_PER_SIMD (kF64 ? CHILD_WAVES_F64 : 4)
 #endif
 #ifndef CHILD_WAVES_F64
-#define CHILD_WAVES_F64 2   // heterogeneous-medium scene, 512^2, 128 spp, nder 3, child kernel per render: 2 waves 413 ms, 4 waves 464 ms (1 wave: 1.5x 2)
+#define CHILD_WAVES_F64 2   // heterogeneous-medium scene, 512^2, 128 spp, nder 3, child kernel per render: 2 waves 194 ms, 3 waves 197, 4 waves 212
 #endif
 // Where the tree lies in HBM a child waits for its nodes one after the other: more waves, at the
-// price of spills. 50K-face dielectric scene, child kernel at 8 lanes 36.7 ms with 2 waves per
+// price of spills. 100K-face dielectric scene, child kernel at 8 lanes 36.7 ms with 2 waves per
 // SIMD, 41.5 with 3, 32.8 with 4, 39.1 with 5; surface scene's tree read from HBM 70.5 -> 62.7 ms.
 #define CHILD_WAVES_HBM 4
 #ifndef AD_WAVES_PER_SIMD
-#define AD_WAVES_PER_SIMD (kF64 ? 1 : 2)   // the surface-only AD kernel and the adjoint
+#define AD_WAVES_PER_SIMD (kF64 ? 1 : 2)   // the surface-only AD kernel
 #endif
 template <int N> constexpr int adWaves() { return N >= 8 ? 1 : AD_WAVES_PER_SIMD; }
 // The staged AD kernels (ad_stages.h): work-groups of four waves, one per SIMD, which share
