@@ -121,15 +121,30 @@ DI void treeToLds(const DScene &S, int lds_nodes, bool lds_tris) {
 // The two children's entry distances (at least tnear) and whether the ray (origin o,
 // reciprocal direction inv) meets their boxes in [tnear, tfar]. n*: the planes it enters
 // by, f*: those it leaves by, each {left, right}. Choosing them by the direction's sign
-// replaces a minimum and a maximum per plane pair; the distances are the same.
+// replaces a minimum and a maximum per plane pair; the distances are the same, but for a ray
+// with a zero direction component whose origin lies in a box plane: there one plane's
+// distance is 0 * inf. in_plane (wave-uniform: some lane's ray has such a component) orders
+// the pairs all the same, and the ray is outside unless the box is flat: about one float
+// camera ray in 65,536 of an odd-sized image's middle column lies in such a plane.
 struct Hit2 { bool l, r; };
+DI void orderPlanes(float2 &n, float2 &f) {
+    const float2 a = n, b = f;
+    n = float2{fminf(a.x, b.x), fminf(a.y, b.y)};
+    f = float2{fmaxf(a.x, b.x), fmaxf(a.y, b.y)};
+}
 DI Hit2 boxesHit(fv3 o, fv3 inv, float2 nx, float2 ny, float2 nz, float2 fx, float2 fy, float2 fz, float tnear, float tfar,
-                 float &tl, float &tr) {
-    tl = fmaxf(fmaxf((nx.x - o.x) * inv.x, (ny.x - o.y) * inv.y), fmaxf((nz.x - o.z) * inv.z, tnear));
-    tr = fmaxf(fmaxf((nx.y - o.x) * inv.x, (ny.y - o.y) * inv.y), fmaxf((nz.y - o.z) * inv.z, tnear));
-    const float ul = fminf(fminf((fx.x - o.x) * inv.x, (fy.x - o.y) * inv.y), fminf((fz.x - o.z) * inv.z, tfar));
-    const float ur = fminf(fminf((fx.y - o.x) * inv.x, (fy.y - o.y) * inv.y), fminf((fz.y - o.z) * inv.z, tfar));
-    return {tl <= ul, tr <= ur};
+                 bool in_plane, float &tl, float &tr) {
+    nx = float2{(nx.x - o.x) * inv.x, (nx.y - o.x) * inv.x}; fx = float2{(fx.x - o.x) * inv.x, (fx.y - o.x) * inv.x};
+    ny = float2{(ny.x - o.y) * inv.y, (ny.y - o.y) * inv.y}; fy = float2{(fy.x - o.y) * inv.y, (fy.y - o.y) * inv.y};
+    nz = float2{(nz.x - o.z) * inv.z, (nz.y - o.z) * inv.z}; fz = float2{(fz.x - o.z) * inv.z, (fz.y - o.z) * inv.z};
+    if (in_plane) {
+        orderPlanes(nx, fx);
+        orderPlanes(ny, fy);
+        orderPlanes(nz, fz);
+    }
+    tl = fmaxf(fmaxf(nx.x, ny.x), fmaxf(nz.x, tnear));
+    tr = fmaxf(fmaxf(nx.y, ny.y), fmaxf(nz.y, tnear));
+    return {tl <= fminf(fminf(fx.x, fy.x), fminf(fz.x, tfar)), tr <= fminf(fminf(fx.y, fy.y), fminf(fz.y, tfar))};
 }
 
 // Where the tree of a kernel's launches is: either place, read by a launch-uniform test (ANY),
@@ -151,6 +166,7 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
     const float BEPS = 1e-6f;
     const fv3 inv{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     const bool ngx = inv.x < 0.f, ngy = inv.y < 0.f, ngz = inv.z < 0.f;   // entered by the high planes
+    const bool in_plane = __any(isinf(inv.x) || isinf(inv.y) || isinf(inv.z));
     float best = tfar;
     const float *lds = ldsTree(stack_depth);
     const float *lx = lds + (ngx ? 2 : 0), *ly = lds + (ngy ? 6 : 4), *lz = lds + (ngz ? 10 : 8);
@@ -192,7 +208,7 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
             }
             float tl, tr;
             nbox += 2;
-            const Hit2 hit = boxesHit(o, inv, nx, ny, nz, fx, fy, fz, tnear, best, tl, tr);
+            const Hit2 hit = boxesHit(o, inv, nx, ny, nz, fx, fy, fz, tnear, best, in_plane, tl, tr);
             const bool hl = hit.l, hr = hit.r;
             const bool right = hr && (!hl || tr < tl);   // the right child is the next node
             top[stride] = right ? cl : cr;   // the other one; above the top unless both are hit
