@@ -23,10 +23,11 @@ template <int N> struct AdSlots {
     size_t n;   // slots
     enum Real { RO = 0, RD = 3 * (N + 1), BETA = 6 * (N + 1), L = 9 * (N + 1), CPDF = 12 * (N + 1), ETHR, EBETA = ETHR + 3,
                 EWI = EBETA + 3, EGN = EWI + 3, ESN = EGN + 3, REALS = ESN + 3 };
-    enum Word { PIX = 0, VIEW, FLAGS, FACE, RBLK, RPOS, RB0, RB1, RB2, RB3, CHILD, SKIP, FAILED, EFLAGS, EFACE, WORDS };
+    enum Word { PIX = 0, VIEW, FLAGS, MED, RBLK, RPOS, RB0, RB1, RB2, RB3, CHILD, SKIP, FAILED, EFLAGS, EFACE, WORDS };
     static constexpr size_t BYTES = REALS * sizeof(real) + WORDS * 4;
     static_assert(REALS == adSlotReals(N) && WORDS == AD_SLOT_WORDS, "adSlotBytes sizes this layout");
-    static constexpr uint32_t RD_CONST = 1u << 31;   // FLAGS: rd has no tangents (none are stored)
+    // FLAGS: depth | mode << 8 | walk << 16, then these; rd has no tangents (none are stored)
+    static constexpr uint32_t SURF = 1u << 18, ADD = 1u << 19, RD_CONST = 1u << 20;
     DI real &r(int k, uint32_t slot) const { return f[(size_t)k * n + slot]; }
     DI uint32_t &u(int k, uint32_t slot) const { return w[(size_t)k * n + slot]; }
     DI f3 ld(int k, uint32_t s) const { return f3{r(k, s), r(k + 1, s), r(k + 2, s)}; }
@@ -324,9 +325,9 @@ DI void adBounce(Tracer<N> &T, const RenderParams &P, const AdSlots<N> &a, uint3
         if (keep) a.stv(AS::RD, slot, rd);
         else a.st(AS::RD, slot, nd);
         a.r(AS::CPDF, slot) = cpdf;
-        a.u(AS::FLAGS, slot) = (uint32_t)(med1 + 1) | (uint32_t)(depth - 1) << 8 | (uint32_t)mode1 << 16 |
-                               (first_only ? 1u : 2u) << 22 | (vol ? 0u : 1u << 24) | (addc ? 1u << 25 : 0u) |
-                               (keep ? 0u : AS::RD_CONST);
+        a.u(AS::MED, slot) = (uint32_t)med1;
+        a.u(AS::FLAGS, slot) = (uint32_t)(depth - 1) | (uint32_t)mode1 << 8 | (first_only ? 1u : 2u) << 16 |
+                               (vol ? 0u : AS::SURF) | (addc ? AS::ADD : 0u) | (keep ? 0u : AS::RD_CONST);
         alive = mode1 != 0;
     }
     if (q.live) {   // one shadow walk for both kinds of event
@@ -386,12 +387,12 @@ DI bool adLoad(const DScene &S, const RenderParams &P, const AdBatch &B, const A
     u.failed_at = a.u(A::FAILED, slot);
     a.ldRng(slot, vw.seed, ls, r);
     const uint32_t fl = a.u(A::FLAGS, slot);
-    st.med = (int)(fl & 255u) - 1;
-    st.depth = (int)(fl >> 8 & 255u);
-    st.mode = (int)(fl >> 16 & 63u);
-    st.walk = (int)(fl >> 22 & 3u);
-    st.walk_surf = (fl >> 24 & 1u) != 0;
-    st.walk_add = (fl >> 25 & 1u) != 0;
+    st.med = (int)a.u(A::MED, slot);
+    st.depth = (int)(fl & 255u);
+    st.mode = (int)(fl >> 8 & (uint32_t)AD_MODES);
+    st.walk = (int)(fl >> 16 & 3u);
+    st.walk_surf = (fl & A::SURF) != 0;
+    st.walk_add = (fl & A::ADD) != 0;
     st.walk_cpdf = a.r(A::CPDF, slot);
     st.ro = a.ldv(A::RO, slot);
     st.rd = fl & A::RD_CONST ? Dv<N>(a.ld(A::RD, slot)) : a.ldv(A::RD, slot);
@@ -529,7 +530,7 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_EDGE_WAVES) void k_ad_edges(DSce
         a.ldRng(slot, vw.seed, ls, r);
         const uint32_t fl = a.u(A::EFLAGS, slot);
         const bool vol = (fl & 1u) != 0;
-        const int depth = (int)(fl >> 1 & 255u), med = (int)(fl >> 9 & 255u) - 1;
+        const int depth = (int)(fl >> 1 & 255u), med = (int)(fl >> 9) - 1;
         const Dv<N> x = a.ldv(A::RO, slot);
         Hit its0;
         const DBsdf *bp = nullptr;

@@ -1401,6 +1401,9 @@ bool Scene::setupViews(int nv, const Camera *const *cams, const dtrt_render_opti
     return true;
 }
 
+// The terms that a render's mode asks for; bits that name none are ignored.
+int adMode(const dtrt_render_options &o) { return (o.mode >= 0 ? o.mode : AD_MODES) & AD_MODES; }
+
 constexpr uint64_t FIRST_CHUNK = uint64_t(1) << 18;  // before the children-per-sample rate is known
 
 // All views in one pass: their AD samples form one global sample space (launched in
@@ -1420,8 +1423,8 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
     RenderParams P{};
     P.ad_kind = ad_kind;
     P.max_bounces = o0.max_bounces; P.sppse = std::max(0, o0.sppse);
-    P.mode = o0.mode >= 0 ? o0.mode : 0x3F; P.ddist = o0.ddist_coeff;
-    if (P.max_bounces < 0 || P.max_bounces > 200) return fail("render: max_bounces out of range");
+    P.mode = adMode(o0); P.ddist = o0.ddist_coeff;
+    if (P.max_bounces < 0 || P.max_bounces > AD_MAX_BOUNCES) return fail("render: max_bounces out of range");
     P.rec_stride = childRecordStride(nder, S.f64 != 0);
     P.ad_block = tune_ad_block;
     P.child_block = tune_child_block;
@@ -1618,7 +1621,7 @@ bool Scene::captureViews(int nv, const Camera *const *cams, const dtrt_render_op
     RenderParams P{};
     const dtrt_render_options &o0 = opts[0];
     P.max_bounces = o0.max_bounces; P.sppse = std::max(0, o0.sppse);
-    P.mode = o0.mode >= 0 ? o0.mode : 0x3F; P.ddist = o0.ddist_coeff;
+    P.mode = adMode(o0); P.ddist = o0.ddist_coeff;
     P.rec_stride = childRecordStride(nder, S.f64 != 0);
     P.ad_block = tune_ad_block;
     P.child_block = tune_child_block;
@@ -1798,7 +1801,7 @@ bool Scene::captureStep(StepArgs &a) {
     const dtrt_render_options &o0 = a.fopts[0];
     P.ad_kind = AD_VOLPATH;
     P.max_bounces = o0.max_bounces; P.sppse = std::max(0, o0.sppse);
-    P.mode = o0.mode >= 0 ? o0.mode : 0x3F; P.ddist = o0.ddist_coeff;
+    P.mode = adMode(o0); P.ddist = o0.ddist_coeff;
     P.rec_stride = childRecordStride(nder, S.f64 != 0);
     P.ad_block = tune_ad_block;
     P.child_block = tune_child_block;
@@ -1995,12 +1998,12 @@ bool Scene::renderAdjointViews(int nv, const Camera *const *cams, const dtrt_ren
     const dtrt_render_options &o = opts[0];
     RenderParams P{};
     P.max_bounces = o.max_bounces; P.sppse = 0;
-    P.mode = (o.mode >= 0 ? o.mode : 0x3F) & (1 | 2 | 8);
+    P.mode = adMode(o) & (1 | 2 | 8);
     P.tree_in_hbm = tree_in_hbm ? 1 : 0;
     P.ddist = 0.f;
     std::vector<dtrt_render_options> ov(opts, opts + nv);
     for (auto &x : ov) {
-        if (x.spp <= 0 || x.max_bounces != o.max_bounces || x.mode != o.mode || x.max_bounces < 0 || x.max_bounces > 200)
+        if (x.spp <= 0 || x.max_bounces != o.max_bounces || x.mode != o.mode || x.max_bounces < 0 || x.max_bounces > AD_MAX_BOUNCES)
             return fail("adjoint: bad options (views must share max_bounces and mode)");
         x.sppe = x.sppe < 0 ? -1 : 0;   // pixel jitter as in the forward render; no primary-edge pass
     }
@@ -2051,7 +2054,7 @@ bool Scene::renderAdjointViews(int nv, const Camera *const *cams, const dtrt_ren
 // 3 PathTracer, 4 DirectIntegrator (each pixel the mean of spp jittered samples);
 // 5 ParticleTracer (100000 * spp light particles, splatted and divided by their count).
 bool Scene::renderPrimal(const dtrt_render_options &o, float *out, bool out_is_device, int integrator) {
-    if (o.spp <= 0 || o.max_bounces < 0 || o.max_bounces > 200) return fail("render: bad options");
+    if (o.spp <= 0 || o.max_bounces < 0 || o.max_bounces > AD_MAX_BOUNCES) return fail("render: bad options");
     if (!afterCaller()) return false;
     RenderParams P{};
     P.max_bounces = integrator == 4 ? 1 : o.max_bounces;

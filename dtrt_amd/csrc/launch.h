@@ -30,7 +30,8 @@ struct RenderParams {
 // every bounce.
 constexpr int AD_SLOT_WORDS = 15;
 constexpr int adSlotReals(int nder) { return 12 * (nder + 1) + 16; }
-constexpr int AD_MAX_BOUNCES = 200;
+constexpr int AD_MAX_BOUNCES = 200;   // the most bounces of a render
+constexpr int AD_MODES = 0x3F;        // the bits of RenderParams::mode that name a term (integratorAD.h:12-24)
 constexpr int AD_CNT = 32;   // words from one counter to the next: a cache line each, since all waves count in them
 constexpr uint64_t adSlotBytes(int nder, bool f64) { return (uint64_t)adSlotReals(nder) * (f64 ? 8 : 4) + AD_SLOT_WORDS * 4 + 12; }
 constexpr uint64_t adStateBytes(int nder, bool f64, uint64_t slots) {

@@ -43,7 +43,7 @@ typedef struct dtrt_render_options {
     int32_t sppe;          /* num_samples_primary_edge (<0: pixel centres, no jitter) */
     int32_t sppse;         /* num_samples_secondary_edge */
     int32_t quiet;
-    int32_t mode;          /* EMode bitmask (integratorAD.h:12-24); -1 = all terms */
+    int32_t mode;          /* EMode bitmask (integratorAD.h:12-24; other bits are ignored); negative = all terms */
     float ddist_coeff;     /* ddistCoeff */
 } dtrt_render_options;
 
