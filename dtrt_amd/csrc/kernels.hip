@@ -835,7 +835,7 @@ __global__ void k_refit(float4 *nodes, const float4 *tris, const int *F, const f
 }
 
 // One view of an L2 image loss sum (I - T)^2 over the value channel: dimg = 2 (I - T),
-// the loss added into *loss (one double atomic per wave).
+// the loss added into *loss, unless loss is null (one double atomic per wave).
 __global__ void k_l2_grad(const float *img, const float *target, float *dimg, uint64_t n, double *loss) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     double e2 = 0.0;
@@ -845,7 +845,7 @@ __global__ void k_l2_grad(const float *img, const float *target, float *dimg, ui
         e2 = (double)e * e;
     }
     for (int off = 32; off > 0; off >>= 1) e2 += __shfl_xor(e2, off);
-    if ((threadIdx.x & 63) == 0 && e2 != 0.0) unsafeAtomicAdd(loss, e2);
+    if (loss && (threadIdx.x & 63) == 0 && e2 != 0.0) unsafeAtomicAdd(loss, e2);
 }
 
 // grad[k] += sum_i dimg[i] * tangent_k[i] for the view image img = [(nder + 1)][n]
