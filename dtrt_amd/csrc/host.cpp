@@ -802,7 +802,7 @@ struct Scene : Obj {
         return renderViews(1, &c, &o, outs, out_is_device, ad_kind);
     }
     bool renderViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, float *const *outs, bool on_device,
-                     int ad_kind = AD_VOLPATH, Bump *pool = nullptr);
+                     int ad_kind = AD_VOLPATH, Bump *pool = nullptr, bool for_capture = false);
     bool primaryEdges(const Camera &c, PECache &out);
     void projectPrimaryEdges(const Camera &cam, std::vector<double> &cdf, std::vector<float> &packed, int &npe,
                              double &pe_sum) const;
@@ -854,7 +854,7 @@ struct Scene : Obj {
         float *dgrid = nullptr;
         double *pgrad = nullptr, *loss = nullptr;
     };
-    bool runStep(StepArgs &a);
+    bool runStep(StepArgs &a, bool for_capture = false);
     bool stepLoss(StepArgs &a, const std::vector<DView> &hv, hipStream_t sm);
     bool captureStep(StepArgs &a);
     int replayStep(const uint64_t *seeds);
@@ -1404,14 +1404,19 @@ bool Scene::setupViews(int nv, const Camera *const *cams, const dtrt_render_opti
 // The terms that a render's mode asks for; bits that name none are ignored.
 int adMode(const dtrt_render_options &o) { return (o.mode >= 0 ? o.mode : AD_MODES) & AD_MODES; }
 
-constexpr uint64_t FIRST_CHUNK = uint64_t(1) << 18;  // before the children-per-sample rate is known
+// Samples of the first chunk, before the children-per-sample rate is known: a small view
+// (128^2 at 16 spp) is one chunk, and the queue's default holds 118 children per sample of it at
+// nder 3 in double (measured rates are about 0.4 times sppse). A schedule that is to be
+// captured may not overflow, for other seeds either: where one that starts so does, or its
+// first chunk fills more of the queue than the next ones aim at, it starts again with the fewer.
+constexpr uint64_t FIRST_CHUNK = uint64_t(1) << 18, FIRST_CHUNK_CAPTURE = uint64_t(1) << 16;
 
 // All views in one pass: their AD samples form one global sample space (launched in
 // the same chunks), their primary-edge samples follow view by view, and each view's
 // pixels occupy their own range of the accumulators. Every view's image equals what
 // a render of that view alone gives (same streams), up to float summation order.
 bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, float *const *outs,
-                        bool out_is_device, int ad_kind, Bump *pool) {
+                        bool out_is_device, int ad_kind, Bump *pool, bool for_capture) {
     if (nv <= 0) return fail("render: no views");
     if (pool && !out_is_device) return fail("render: the scratch-only render writes device images only");
     if (!afterCaller()) return false;
@@ -1494,10 +1499,14 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
     // clears by fill kernels (the scratch area keeps the last call's contents)
-    HIPCHK(launch_fill32(A, img * es / 4, 0u, stream));
-    HIPCHK(launch_fill32(APE, (size_t)nder * npix * 3 * es / 4, 0u, stream));
-    HIPCHK(launch_fill32(st, 64, 0u, stream));
-    HIPCHK(launch_fill32(wk, 32, 0u, stream));
+    auto clear = [&]() -> bool {
+        HIPCHK(launch_fill32(A, img * es / 4, 0u, stream));
+        HIPCHK(launch_fill32(APE, (size_t)nder * npix * 3 * es / 4, 0u, stream));
+        HIPCHK(launch_fill32(st, 64, 0u, stream));
+        HIPCHK(launch_fill32(wk, 32, 0u, stream));
+        return true;
+    };
+    if (!clear()) return false;
     // per-view output images in device memory (staged through outbuf for host outputs)
     std::vector<float *> dout(nv);
     if (out_is_device) {
@@ -1555,6 +1564,14 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
         if (!timed(0, [&] { return launch_ad_paths(S, P, s0, n, nullptr, A, Q, qc, st, OV[0], qc + 1, wk, stream); })) return false;
         if (!timed(1, [&] { return launch_children(S, P, Q, qc, A, APE, wk, childGrid, stream); })) return false;
         if (!counts(h)) return false;
+        const bool tight = h[1] > 0 || (last_chunks.size() == 1 && (double)h[0] > tune_fill * (double)cap);
+        if (for_capture && tight && last_chunks.front() > FIRST_CHUNK_CAPTURE) {   // no image is written yet
+            if (!clear()) return false;
+            last_chunks.clear();
+            children = s0 = 0;
+            chunk = FIRST_CHUNK_CAPTURE;
+            continue;
+        }
         delivered += std::min<uint64_t>(h[0], cap);
         int in = 0;
         for (unsigned nov = h[1]; nov > 0; in ^= 1) {   // each round delivers >= 1 record: terminates
@@ -1616,7 +1633,7 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
 // path, so a replay is always exact.
 bool Scene::captureViews(int nv, const Camera *const *cams, const dtrt_render_options *opts, float *const *images) {
     graph.reset();
-    if (!renderViews(nv, cams, opts, images, true)) return false;
+    if (!renderViews(nv, cams, opts, images, true, AD_VOLPATH, nullptr, true)) return false;
     if (last_replayed) return fail("capture: the schedule overflowed the child queue; render in smaller batches");
     RenderParams P{};
     const dtrt_render_options &o0 = opts[0];
@@ -1759,7 +1776,7 @@ static bool stepOptionsValid(const Scene::StepArgs &a) {
     return true;
 }
 
-bool Scene::runStep(StepArgs &a) {
+bool Scene::runStep(StepArgs &a, bool for_capture) {
     const int nv = (int)a.cams.size();
     if (!gridMedium(a.med) || !a.dgrid) return false;
     if (!stepOptionsValid(a)) return false;
@@ -1771,7 +1788,7 @@ bool Scene::runStep(StepArgs &a) {
         const uint64_t np = c.cropped() ? (uint64_t)c.cw * c.ch : (uint64_t)c.w * c.h;
         HIPCHK(launch_fill32(a.images[v], (uint64_t)(nder + 1) * np * 3, 0u, stream));
     }
-    if (!renderViews(nv, cp.data(), a.fopts.data(), a.images.data(), true)) return false;
+    if (!renderViews(nv, cp.data(), a.fopts.data(), a.images.data(), true, AD_VOLPATH, nullptr, for_capture)) return false;
     std::vector<DView> hv;
     std::vector<uint64_t> pe_total;
     if (!setupViews(nv, cp.data(), a.fopts.data(), hv, pe_total)) return false;
@@ -1792,7 +1809,7 @@ bool Scene::runStep(StepArgs &a) {
 // table in viewbuf, the adjoint's lies in stepbuf, so replays rewrite both.
 bool Scene::captureStep(StepArgs &a) {
     stepg.reset();
-    if (!runStep(a)) return false;
+    if (!runStep(a, true)) return false;
     if (last_replayed) return fail("capture_step: the schedule overflowed the child queue; render in smaller batches");
     const int nv = (int)a.cams.size();
     std::vector<const Camera *> cp;
