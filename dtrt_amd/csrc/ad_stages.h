@@ -7,7 +7,7 @@
 //  k_ad_edges<N>    the edge term (edgeTerm) of the bounces that have one
 //  k_ad_finish<N>   the samples' radiance into the accumulators, the samples whose pushes
 //                   overflowed the queue into the replay list
-//  k_adj_list<N>, k_adj_bounce<N>
+//  k_adj_list<1>, k_adj_bounce<1>
 //                   the density adjoint: which samples take part, and the bounces of the
 //                   replay that scatters the derivative of every contribution
 //

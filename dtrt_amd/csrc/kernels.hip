@@ -6,7 +6,7 @@
 //                   paths still alive. They sum the interior terms and push every primal
 //                   sub-path the boundary terms need (2 per accepted edge sample, 1 per
 //                   Lins sample) into an HBM queue.
-//  k_adj_list<N>, k_adj_bounce<N> (ad_stages.h)
+//  k_adj_list<1>, k_adj_bounce<1> (ad_stages.h)
 //                   the density adjoint's replay of those paths.
 //  k_ad_paths<N>    the same for the surface-only integrators, one thread per sample.
 //  k_children<N>    one thread per queued sub-path: primal Li / Lins estimate, scattered
@@ -1289,8 +1289,16 @@ template <int N> struct WidthOps {
     static void launchFinalize(const RenderParams &P, int npix, int pix0, int spp, int has_pe, const real *acc,
                                const real *acc_pe, float *out, unsigned *st, hipStream_t sm);
     static void launchGrid(const DScene &S, int med, const float *pts, int n, float *out, hipStream_t sm);
-    static void launchAdjoint(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg,
-                              double *grad, int pmed, unsigned *st, unsigned long long *wk, hipStream_t sm);
+    static hipError_t kernelInfo(KernelInfo *out, int cap, int *count);
+};
+// The density adjoint, whose kernels are those of one lane at every scene's width (defined in
+// the object of width 1): the density derivatives come from the scattered values, no tangent
+// enters them, and a value does not depend on the lanes. The scene's tangents are then read at a
+// narrower stride than the scene's arrays have: in bounds, and unused. A step of the
+// dielectric scene at 8 lanes, 73K samples: adjoint 19.5 ms at the scene's width, 11.0 ms at one lane.
+struct AdjointOps {
+    static void launch(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg, double *grad, int pmed,
+                       unsigned *st, unsigned long long *wk, hipStream_t sm);
     static hipError_t kernelInfo(KernelInfo *out, int cap, int *count);
 };
 
@@ -1455,43 +1463,6 @@ template <int N> void WidthOps<N>::launchAdStages(const DScene &S, const RenderP
         hipLaunchKernelGGL(k_ad_finish<N>, dim3((B.m + 255) / 256, 3 * (N + 1)), dim3(256), 0, sm, P, B, acc, ovf, ovf_count);
     }
 }
-// The density adjoint of a chunk, batch by batch: the radiance of every sample whose pixel
-// has a loss gradient (k_ad_bounce, without edge terms), then k_adj_bounce over those
-// that have any.
-template <int N> void WidthOps<N>::launchAdjoint(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n,
-                                                 const float *dimg, double *grad, int pmed, unsigned *st,
-                                                 unsigned long long *wk, hipStream_t sm) {
-    const unsigned blk = AD_STAGE_BLOCK, wpb = blk / 64;
-    RenderParams Pb = P, Pa = P;
-    const size_t lb = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_bounce<N>, blk, S, Pb, treePrefixInLds<N>());
-    const size_t la = traceLds(blk, S.stack_depth) + treeLdsFor(k_adj_bounce<N>, blk, S, Pa, treePrefixInLds<N>());
-    const unsigned rb = residentBlocks(k_ad_bounce<N>, blk, lb), ra = residentBlocks(k_adj_bounce<N>, blk, la);
-    const AdLists ls(P, AdSlots<N>::BYTES);
-    AdBatch B{};
-    B.state = P.ad_state;
-    B.n = P.ad_slots;
-    for (uint64_t b0 = 0; b0 < n; b0 += B.n) {
-        B.m = (uint32_t)std::min<uint64_t>(B.n, n - b0);
-        B.s0 = s0 + b0;
-        const unsigned few = (B.m + 4 * wpb - 1) / (4 * wpb);
-        for (int pass = 0; pass < 2; ++pass) {
-            (void)launch_fill32(ls.cnt, 4 * (P.max_bounces + 3) * AD_CNT, 0u, sm);
-            B.out = ls.alive[0];
-            B.cnt = ls.cnt;
-            hipLaunchKernelGGL(k_adj_list<N>, dim3((B.m + 255) / 256), dim3(256), 0, sm, S, B, dimg, pass);
-            for (int k = 0; k <= P.max_bounces; ++k) {
-                B.start = k == 0;
-                B.in = ls.alive[k & 1];
-                B.out = ls.alive[(k + 1) & 1];
-                B.cnt = ls.cnt + 4 * k * AD_CNT;
-                if (pass == 0)
-                    hipLaunchKernelGGL(k_ad_bounce<N>, dim3(std::min(rb, few)), dim3(blk), lb, sm, S, Pb, B, nullptr, nullptr, st, wk);
-                else
-                    hipLaunchKernelGGL(k_adj_bounce<N>, dim3(std::min(ra, few)), dim3(blk), la, sm, S, Pa, B, grad, pmed, st, wk);
-            }
-        }
-    }
-}
 template <int N> void WidthOps<N>::launchChildren(const DScene &S, const RenderParams &P, const char *q, unsigned *qc,
                                             real *acc, real *acc_pe, unsigned long long *wk, unsigned grid, hipStream_t sm) {
     // grid: the most blocks of the default size; no more than the device holds at once are
@@ -1548,14 +1519,60 @@ template <int N> hipError_t WidthOps<N>::kernelInfo(KernelInfo *out, int cap, in
     DT_INFO((k_children_path<N, Tree::LDS>), "k_children_path", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_children_path<N, Tree::HBM>), "k_children_path/hbm", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO(k_primary<N>, "k_primary", PRIMARY_BLOCK, traceLds(PRIMARY_BLOCK))
-    DT_INFO(k_adj_bounce<N>, "k_adj_bounce", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
-    DT_INFO(k_adj_list<N>, "k_adj_list", 256, 0)
     DT_INFO(k_grid<N>, "k_grid", BLOCK, 0)
     DT_INFO(k_finalize<N>, "k_finalize", 256, 0)
 #undef DT_INFO
     return e;
 }
 template struct WidthOps<DT_N>;
+
+#if DT_N == 1
+// The density adjoint of a chunk, batch by batch: the radiance of every sample whose pixel
+// has a loss gradient (k_ad_bounce, without edge terms), then k_adj_bounce over those
+// that have any.
+void AdjointOps::launch(const DScene &S_, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg, double *grad, int pmed,
+                        unsigned *st, unsigned long long *wk, hipStream_t sm) {
+    constexpr int N = 1;
+    DScene S = S_;
+    S.nder = N;
+    const unsigned blk = AD_STAGE_BLOCK, wpb = blk / 64;
+    RenderParams Pb = P, Pa = P;
+    const size_t lb = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_bounce<N>, blk, S, Pb, treePrefixInLds<N>());
+    const size_t la = traceLds(blk, S.stack_depth) + treeLdsFor(k_adj_bounce<N>, blk, S, Pa, treePrefixInLds<N>());
+    const unsigned rb = residentBlocks(k_ad_bounce<N>, blk, lb), ra = residentBlocks(k_adj_bounce<N>, blk, la);
+    const AdLists ls(P, AdSlots<N>::BYTES);
+    AdBatch B{};
+    B.state = P.ad_state;
+    B.n = P.ad_slots;
+    for (uint64_t b0 = 0; b0 < n; b0 += B.n) {
+        B.m = (uint32_t)std::min<uint64_t>(B.n, n - b0);
+        B.s0 = s0 + b0;
+        const unsigned few = (B.m + 4 * wpb - 1) / (4 * wpb);
+        for (int pass = 0; pass < 2; ++pass) {
+            (void)launch_fill32(ls.cnt, 4 * (P.max_bounces + 3) * AD_CNT, 0u, sm);
+            B.out = ls.alive[0];
+            B.cnt = ls.cnt;
+            hipLaunchKernelGGL(k_adj_list<N>, dim3((B.m + 255) / 256), dim3(256), 0, sm, S, B, dimg, pass);
+            for (int k = 0; k <= P.max_bounces; ++k) {
+                B.start = k == 0;
+                B.in = ls.alive[k & 1];
+                B.out = ls.alive[(k + 1) & 1];
+                B.cnt = ls.cnt + 4 * k * AD_CNT;
+                if (pass == 0)
+                    hipLaunchKernelGGL(k_ad_bounce<N>, dim3(std::min(rb, few)), dim3(blk), lb, sm, S, Pb, B, nullptr, nullptr, st, wk);
+                else
+                    hipLaunchKernelGGL(k_adj_bounce<N>, dim3(std::min(ra, few)), dim3(blk), la, sm, S, Pa, B, grad, pmed, st, wk);
+            }
+        }
+    }
+}
+hipError_t AdjointOps::kernelInfo(KernelInfo *out, int cap, int *count) {
+    hipError_t e = addKernelInfo(k_ad_bounce<1>, "k_ad_bounce<1>/adjoint", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_adj_bounce<1>, "k_adj_bounce<1>", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_adj_list<1>, "k_adj_list<1>", 256, 0, out, cap, count);
+    return e;
+}
+#endif
 
 #else  // the width-independent object of this precision: dispatchers over S.nder and the remaining launchers
 
@@ -1597,14 +1614,7 @@ hipError_t launch_primary(const DScene &S, const RenderParams &P, int view, uint
 }
 hipError_t launch_adjoint(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, const float *dimg, double *grad,
                           int pmed, unsigned *st, unsigned long long *wk, hipStream_t sm) {
-    // At every scene's width the kernels of one lane: the density derivatives come from the
-    // scattered values, no tangent enters them, and a value does not depend on the lanes (the
-    // one lane's tangents are then of a narrower stride than the scene's arrays: in bounds,
-    // and unused). A step of the dielectric scene at 8 lanes, 73K samples: adjoint 19.5 ms at
-    // the scene's width, 11.0 ms at one lane.
-    DScene S1 = S;
-    S1.nder = 1;
-    WidthOps<1>::launchAdjoint(S1, P, s0, n, dimg, grad, pmed, st, wk, sm);
+    AdjointOps::launch(S, P, s0, n, dimg, grad, pmed, st, wk, sm);
     return hipGetLastError();
 }
 hipError_t launch_fill32(void *p, uint64_t n, uint32_t v, hipStream_t sm) {
@@ -1723,6 +1733,7 @@ hipError_t kernel_info(const DScene &S, KernelInfo *out, int cap, int *count) {
 #undef DT_INFO_N
         default: return hipErrorInvalidValue;
     }
+    if (e == hipSuccess) e = AdjointOps::kernelInfo(out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::LDS>, "k_primal_paths/volpath", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::HBM>, "k_primal_paths/volpath/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE, Tree::LDS>, "k_primal_paths/simple", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
