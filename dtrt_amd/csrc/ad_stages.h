@@ -5,6 +5,8 @@
 //                   that the last bounce handed over first; the first launch of a batch
 //                   starts the samples at their camera rays
 //  k_ad_edges<N>    the edge term (edgeTerm) of the bounces that have one
+//  k_ad_tail<N>     the paths of a list too short to fill the chip, from where they are to
+//                   their ends
 //  k_ad_finish<N>   the samples' radiance into the accumulators, the samples whose pushes
 //                   overflowed the queue into the replay list
 //  k_adj_list<1>, k_adj_bounce<1>
@@ -81,6 +83,7 @@ struct AdBatch {
     const uint32_t *in;          // slots alive at the start of the bounce (nullptr: all m)
     uint32_t *out, *edges;       // slots alive after it; slots with an edge term
     uint32_t *cnt;               // AD_CNT words apart: length of in, consumed, length of edges, consumed, length of out
+    uint32_t tail;               // lists of at most so many paths are k_ad_tail's
 };
 template <int N> DI AdSlots<N> slotsOf(const AdBatch &B) {
     AdSlots<N> a;
@@ -348,11 +351,11 @@ DI void adBounce(Tracer<N> &T, const RenderParams &P, const AdSlots<N> &a, uint3
     }
 }
 
-// The path of `slot` at the start of a bounce: its camera ray (B.start) or its stored state.
+// The path of `slot` at the start of a bounce: its camera ray (start) or its stored state.
 // False when it has nothing to do.
 template <int N>
-DI bool adLoad(const DScene &S, const RenderParams &P, const AdBatch &B, const AdSlots<N> &a, uint32_t slot, Rng &r, AdState<N> &st,
-               Pusher &u) {
+DI bool adLoad(const DScene &S, const RenderParams &P, const AdBatch &B, const AdSlots<N> &a, uint32_t slot, bool start, Rng &r,
+               AdState<N> &st, Pusher &u) {
     using A = AdSlots<N>;
     uint64_t sid = B.s0 + slot;
     if (B.replay) {
@@ -360,11 +363,11 @@ DI bool adLoad(const DScene &S, const RenderParams &P, const AdBatch &B, const A
         sid = (uint64_t)e.x | ((uint64_t)e.y << 32);
         u.skip = e.z;
     }
-    u.view = B.start ? viewOf(S, sid) : (int)a.u(A::VIEW, slot);
+    u.view = start ? viewOf(S, sid) : (int)a.u(A::VIEW, slot);
     const DView &vw = S.views[u.view];
     const uint64_t ls = sid - vw.s0;   // sample index within the view: keys its random stream
     u.key = (ls + 1) << 20;
-    if (B.start) {
+    if (start) {
         const int pixel = (int)(ls / (uint64_t)vw.spp);
         u.gpix = vw.pix0 + pixel;
         a.u(A::PIX, slot) = (uint32_t)u.gpix;
@@ -405,7 +408,9 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_ad_bounce(D
                                                                              unsigned long long *work) {
     using A = AdSlots<N>;
     const A a = slotsOf<N>(B);
-    ListShare share(B.cnt + AD_CNT, B.in ? B.cnt[0] : B.m);
+    const uint32_t n = B.in ? B.cnt[0] : B.m;
+    if (n <= B.tail) return;
+    ListShare share(B.cnt + AD_CNT, n);
     if (share.idleBlock()) return;
     Tracer<N> T(S);
     T.useLdsTree(P);
@@ -418,7 +423,7 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_ad_bounce(D
             AdState<N> st;
             Rng r;
             Pusher u{q, qcount, 0, 0, 0, 0, 0, Pusher::NO_FAIL};
-            if (adLoad<N>(S, P, B, a, slot, r, st, u))
+            if (adLoad<N>(S, P, B, a, slot, B.start, r, st, u))
                 adBounce<N, AdPass::FORWARD>(T, P, a, slot, r, st, u, stats, nullptr, alive, edge);
             nlk += r.nlk;
             a.u(A::CHILD, slot) = u.child;
@@ -475,7 +480,9 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_adj_bounce(
                                                                               unsigned long long *work) {
     using A = AdSlots<N>;
     const A a = slotsOf<N>(B);
-    ListShare share(B.cnt + AD_CNT, B.cnt[0]);
+    const uint32_t n = B.cnt[0];
+    if (n <= B.tail) return;
+    ListShare share(B.cnt + AD_CNT, n);
     if (share.idleBlock()) return;
     Tracer<N> T(S);
     T.useLdsTree(P);
@@ -489,7 +496,7 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_adj_bounce(
             Rng r;
             Pusher u{nullptr, nullptr, 0, 0, 0, 0, 0, Pusher::NO_FAIL};
             const AdjCtx ac{grad, S.media + pmed, a.ld(A::EBETA, slot), a.ld(A::ETHR, slot)};
-            if (adLoad<N>(S, P, B, a, slot, r, st, u))
+            if (adLoad<N>(S, P, B, a, slot, B.start, r, st, u))
                 adBounce<N, AdPass::SCATTER>(T, P, a, slot, r, st, u, stats, &ac, alive, edge);
             nlk += r.nlk;
             if (alive) a.stRng(slot, r);
@@ -499,14 +506,55 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_BOUNCE_WAVES) void k_adj_bounce(
     flushWork(work, 0, T.nbox, T.ntri, nlk, T.nseg);
 }
 
-// The edge terms of one bounce. The random stream and the child count continue from the
-// bounce's and are handed on to the next one.
+// The edge term of the bounce that the path of `slot` has just made. The random stream and
+// the child count continue from the bounce's and are handed on to the next one.
+template <int N>
+DI void adEdge(Tracer<N> &T, const RenderParams &P, const AdBatch &B, const AdSlots<N> &a, uint32_t slot, char *q, unsigned *qcount,
+               unsigned *stats, uint32_t &nlk) {
+    using A = AdSlots<N>;
+    const DScene &S = T.S;
+    uint64_t sid = B.s0 + slot;
+    if (B.replay) {
+        const uint4 e = B.replay[slot];
+        sid = (uint64_t)e.x | ((uint64_t)e.y << 32);
+    }
+    const int view = (int)a.u(A::VIEW, slot);
+    const DView &vw = S.views[view];
+    const uint64_t ls = sid - vw.s0;
+    Pusher u{q, qcount, (int)a.u(A::PIX, slot), view, (ls + 1) << 20, a.u(A::CHILD, slot), a.u(A::SKIP, slot), a.u(A::FAILED, slot)};
+    Rng r;
+    a.ldRng(slot, vw.seed, ls, r);
+    const uint32_t fl = a.u(A::EFLAGS, slot);
+    const bool vol = (fl & 1u) != 0;
+    const int depth = (int)(fl >> 1 & 255u), med = (int)(fl >> 9) - 1;
+    const Dv<N> x = a.ldv(A::RO, slot);
+    Hit its0;
+    const DBsdf *bp = nullptr;
+    const DPhase *ph = nullptr;
+    f3 rdin{0, 0, 0};
+    if (vol) {
+        ph = &S.phases[S.media[med].phase_id];
+        rdin = a.ld(A::EWI, slot);
+    } else {
+        its0.face = (int)a.u(A::EFACE, slot);
+        its0.p = x.val();
+        its0.wi = a.ld(A::EWI, slot);
+        its0.gn = a.ld(A::EGN, slot);
+        its0.sn = a.ld(A::ESN, slot);
+        bp = &bsdfOf(S, shapeOf(S, its0.face));
+    }
+    edgeTerm<N>(T, P, r, vol, x, &its0, bp, ph, rdin, a.ld(A::ETHR, slot), a.ld(A::EBETA, slot), med, depth, u, stats);
+    nlk += r.nlk;
+    a.stRng(slot, r);
+    a.u(A::CHILD, slot) = u.child;
+    a.u(A::FAILED, slot) = u.failed_at;
+}
+// The edge terms of one bounce.
 template <int N>
 __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_EDGE_WAVES) void k_ad_edges(DScene S, RenderParams P, AdBatch B, char *q,
                                                                           unsigned *qcount, unsigned *stats,
                                                                           unsigned long long *work) {
-    using A = AdSlots<N>;
-    const A a = slotsOf<N>(B);
+    const AdSlots<N> a = slotsOf<N>(B);
     ListShare share(B.cnt + 3 * AD_CNT, B.cnt[2 * AD_CNT]);
     if (share.idleBlock()) return;
     Tracer<N> T(S);
@@ -514,44 +562,66 @@ __global__ __launch_bounds__(AD_STAGE_BLOCK, AD_EDGE_WAVES) void k_ad_edges(DSce
     uint32_t nlk = 0;
     for (; share.more(); share.next()) {
         uint32_t li;
-        if (share.item(li)) {
-        const uint32_t slot = B.edges[li];
-        uint64_t sid = B.s0 + slot;
-        if (B.replay) {
-            const uint4 e = B.replay[slot];
-            sid = (uint64_t)e.x | ((uint64_t)e.y << 32);
+        if (share.item(li)) adEdge<N>(T, P, B, a, B.edges[li], q, qcount, stats, nlk);
+    }
+    flushWork(work, 0, T.nbox, T.ntri, nlk, T.nseg);
+}
+
+// The paths of the batch's short list, if it has one (at most B.tail paths), to their ends: a
+// launch per bounce waits for the slowest path of every bounce, one launch for the slowest
+// path. A bounce that finds its list so short leaves it, and all later lists are empty: it is the
+// last one with any path. B.in, B.out: the lists of even and odd bounces; B.cnt: the
+// counters of bounce 0; B.start: the list is the whole batch, and no bounce has run.
+template <int N, AdPass A, bool EDGES>
+__global__ __launch_bounds__(AD_STAGE_BLOCK, AD_TAIL_WAVES) void k_ad_tail(DScene S, RenderParams P, AdBatch B, char *q,
+                                                                         unsigned *qcount, double *grad, int pmed,
+                                                                         unsigned *stats, unsigned long long *work) {
+    using AS = AdSlots<N>;
+    const AS a = slotsOf<N>(B);
+    uint32_t n = B.m;
+    int at = 0;   // the list's bounce
+    if (!B.start) {
+        n = 0;
+        const int lane = threadIdx.x & 63;
+        for (int k0 = 0; k0 <= P.max_bounces; k0 += 64) {
+            const uint32_t c = k0 + lane <= P.max_bounces ? B.cnt[4 * (k0 + lane) * AD_CNT] : 0;
+            const uint64_t some = __ballot(c > 0);
+            if (!some) continue;
+            const int last = 63 - __clzll(some);
+            at = k0 + last;
+            n = __shfl(c, last);
         }
-        const int view = (int)a.u(A::VIEW, slot);
-        const DView &vw = S.views[view];
-        const uint64_t ls = sid - vw.s0;
-        Pusher u{q, qcount, (int)a.u(A::PIX, slot), view, (ls + 1) << 20, a.u(A::CHILD, slot), a.u(A::SKIP, slot),
-                 a.u(A::FAILED, slot)};
-        Rng r;
-        a.ldRng(slot, vw.seed, ls, r);
-        const uint32_t fl = a.u(A::EFLAGS, slot);
-        const bool vol = (fl & 1u) != 0;
-        const int depth = (int)(fl >> 1 & 255u), med = (int)(fl >> 9) - 1;
-        const Dv<N> x = a.ldv(A::RO, slot);
-        Hit its0;
-        const DBsdf *bp = nullptr;
-        const DPhase *ph = nullptr;
-        f3 rdin{0, 0, 0};
-        if (vol) {
-            ph = &S.phases[S.media[med].phase_id];
-            rdin = a.ld(A::EWI, slot);
-        } else {
-            its0.face = (int)a.u(A::EFACE, slot);
-            its0.p = x.val();
-            its0.wi = a.ld(A::EWI, slot);
-            its0.gn = a.ld(A::EGN, slot);
-            its0.sn = a.ld(A::ESN, slot);
-            bp = &bsdfOf(S, shapeOf(S, its0.face));
-        }
-        edgeTerm<N>(T, P, r, vol, x, &its0, bp, ph, rdin, a.ld(A::ETHR, slot), a.ld(A::EBETA, slot), med, depth, u, stats);
-        nlk += r.nlk;
-        a.stRng(slot, r);
-        a.u(A::CHILD, slot) = u.child;
-        a.u(A::FAILED, slot) = u.failed_at;
+    }
+    if (n > B.tail) return;
+    ListShare share(B.cnt + 4 * (P.max_bounces + 2) * AD_CNT, n);
+    if (share.idleBlock()) return;
+    const uint32_t *list = B.start ? nullptr : at & 1 ? B.out : B.in;
+    Tracer<N> T(S);
+    T.useLdsTree(P);
+    uint32_t nlk = 0;
+    for (; share.more(); share.next()) {
+        uint32_t li;
+        if (!share.item(li)) continue;
+        const uint32_t slot = list ? list[li] : li;
+        bool alive = true, edge;
+        for (bool start = at == 0; alive; start = false) {
+            alive = edge = false;
+            AdState<N> st;
+            Rng r;
+            Pusher u{q, qcount, 0, 0, 0, 0, 0, Pusher::NO_FAIL};
+            const bool go = adLoad<N>(S, P, B, a, slot, start, r, st, u);
+            if constexpr (A == AdPass::FORWARD) {
+                if (go) adBounce<N, A>(T, P, a, slot, r, st, u, stats, nullptr, alive, edge);
+                a.u(AS::CHILD, slot) = u.child;
+                a.u(AS::FAILED, slot) = u.failed_at;
+            } else {
+                const AdjCtx ac{grad, S.media + pmed, a.ld(AS::EBETA, slot), a.ld(AS::ETHR, slot)};
+                if (go) adBounce<N, A>(T, P, a, slot, r, st, u, stats, &ac, alive, edge);
+            }
+            nlk += r.nlk;
+            if (alive || edge) a.stRng(slot, r);
+            if constexpr (EDGES)
+                if (edge) adEdge<N>(T, P, B, a, slot, q, qcount, stats, nlk);
         }
     }
     flushWork(work, 0, T.nbox, T.ntri, nlk, T.nseg);

@@ -671,6 +671,12 @@ constexpr uint64_t NOALLOC_MIN_QUEUE = uint64_t(16) << 20;
 #define AD_SLOTS_LOG 22
 #endif
 constexpr uint64_t AD_SLOTS = uint64_t(1) << AD_SLOTS_LOG;
+// Lists of at most so many paths run to their ends in one launch (k_ad_tail): as many as the
+// device holds at one wave per SIMD. Bounce by bounce such a list waits for its slowest path at
+// every bounce: density gradient of 64^2 at 16 spp and 10 bounces 5.05 ms, with tails 4.08; 8-lane
+// dielectric scene of 25K faces, 64^2 at 16 spp, 200 bounces 92 -> 80 ms. Longer lists lose more
+// by their waves' idle lanes (100K faces, 192^2 at 16 spp: 66.2 ms at this line, 82.2 at 2^18).
+constexpr unsigned AD_TAIL = 1u << 16;
 
 struct Scene : Obj {
     Scene() : Obj(T_SCENE) {}
@@ -756,6 +762,10 @@ struct Scene : Obj {
     // 262 -> 220 ms in float, against 64.
     int tune_ad_block = 64, tune_child_block = 256;
     DevBuf tunebuf;
+    // test settings: of AD_SLOTS, of AD_TAIL, and the most slots that can be allocated
+    int test_ad_slots = 0, test_ad_tail = -1, test_ad_alloc = INT_MAX;
+    unsigned adSlots() const { return test_ad_slots > 0 ? (unsigned)test_ad_slots : (unsigned)AD_SLOTS; }
+    unsigned adTail() const { return test_ad_tail >= 0 ? (unsigned)test_ad_tail : AD_TAIL; }
     // The path state of the staged AD kernels for chunks of up to `chunk` samples of `lanes`
     // lanes, or for fewer at once: where memory is short, and where a larger one would take
     // the buffers away from a captured graph that can be replayed.
@@ -764,7 +774,7 @@ struct Scene : Obj {
         if (a.tried < want && !(a.slots && replayable())) {
             a.tried = want;
             a.slots = 0;
-            while (!ensure(a.b, adStateBytes(lanes, S.f64 != 0, want))) {
+            while (want > (unsigned)test_ad_alloc || !ensure(a.b, adStateBytes(lanes, S.f64 != 0, want))) {
                 (void)hipGetLastError();
                 if (want <= 1u << 16) { a.tried = 0; return false; }
                 want = want / 2 / 64 * 64;
@@ -772,7 +782,7 @@ struct Scene : Obj {
             a.slots = want;
         }
         P.ad_state = static_cast<char *>(a.b.p);
-        P.ad_slots = a.slots;
+        P.ad_slots = std::min(a.slots, adSlots());
         return true;
     }
     // The adjoint's kernels run at one lane (launch_adjoint).
@@ -1434,6 +1444,8 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
     P.ad_block = tune_ad_block;
     P.child_block = tune_child_block;
     P.tree_in_hbm = tree_in_hbm ? 1 : 0;
+    P.ad_tail = adTail();
+    P.ad_ask = 1;
     std::vector<DView> hv;
     std::vector<uint64_t> pe_total;
     if (!setupViews(nv, cams, opts, hv, pe_total, pool)) return false;
@@ -1474,7 +1486,7 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
                         std::to_string((img + (size_t)nder * npix * 3) * es >> 20) + " MiB, plus a queue of at least " +
                         std::to_string(NOALLOC_MIN_QUEUE >> 20) + " MiB)");
         // a quarter of it for the path state, as many samples in flight as fit
-        P.ad_slots = (unsigned)std::min<uint64_t>(AD_SLOTS, (qbytes / 4 - adStateBytes(nder, S.f64 != 0, 0)) / adSlotBytes(nder, S.f64 != 0) / 64 * 64);
+        P.ad_slots = (unsigned)std::min<uint64_t>(adSlots(), (qbytes / 4 - adStateBytes(nder, S.f64 != 0, 0)) / adSlotBytes(nder, S.f64 != 0) / 64 * 64);
         P.ad_state = static_cast<char *>(pool->take(adStateBytes(nder, S.f64 != 0, P.ad_slots)));
         const uint64_t qleft = pool->left / 256 * 256;
         Q = static_cast<char *>(pool->take(qleft));
@@ -1643,6 +1655,7 @@ bool Scene::captureViews(int nv, const Camera *const *cams, const dtrt_render_op
     P.ad_block = tune_ad_block;
     P.child_block = tune_child_block;
     P.tree_in_hbm = tree_in_hbm ? 1 : 0;
+    P.ad_tail = adTail();
     std::vector<DView> hv;
     std::vector<uint64_t> pe_total;
     if (!setupViews(nv, cams, opts, hv, pe_total)) return false;
@@ -1655,7 +1668,7 @@ bool Scene::captureViews(int nv, const Camera *const *cams, const dtrt_render_op
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
     P.ad_state = static_cast<char *>(adstate.b.p);
-    P.ad_slots = adstate.slots;
+    P.ad_slots = std::min(adstate.slots, adSlots());
     int dev = 0, ncu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -1823,6 +1836,7 @@ bool Scene::captureStep(StepArgs &a) {
     P.ad_block = tune_ad_block;
     P.child_block = tune_child_block;
     P.tree_in_hbm = tree_in_hbm ? 1 : 0;
+    P.ad_tail = adTail();
     std::vector<DView> hvf, hva;
     std::vector<uint64_t> pe_total, pe_unused;
     if (!setupViews(nv, cp.data(), a.fopts.data(), hvf, pe_total)) return false;
@@ -1847,7 +1861,7 @@ bool Scene::captureStep(StepArgs &a) {
     const uint64_t pe_chunk = std::max<uint64_t>(64, std::min<uint64_t>(cap / 2 / 64 * 64, uint64_t(1) << 23));
     P.qcap = (unsigned)cap;
     P.ad_state = static_cast<char *>(adstate.b.p);
-    P.ad_slots = adstate.slots;
+    P.ad_slots = std::min(adstate.slots, adSlots());
     int dev = 0, ncu = 0;
     HIPCHK(hipGetDevice(&dev));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -2017,6 +2031,8 @@ bool Scene::renderAdjointViews(int nv, const Camera *const *cams, const dtrt_ren
     P.max_bounces = o.max_bounces; P.sppse = 0;
     P.mode = adMode(o) & (1 | 2 | 8);
     P.tree_in_hbm = tree_in_hbm ? 1 : 0;
+    P.ad_tail = adTail();
+    P.ad_ask = launch;
     P.ddist = 0.f;
     std::vector<dtrt_render_options> ov(opts, opts + nv);
     for (auto &x : ov) {
@@ -2860,6 +2876,17 @@ int dtrt_test_set_tree_in_hbm(dtrt_object *scene, int on) {
         Scene *s = as<Scene>(scene, T_SCENE);
         if (!s) return -1;
         s->tree_in_hbm = on != 0;
+        return 0;
+    });
+}
+
+int dtrt_test_set_ad_batch(dtrt_object *scene, int slots, int tail, int alloc_slots) {
+    return guarded<int>(-1, [&]() -> int {
+        Scene *s = as<Scene>(scene, T_SCENE);
+        if (!s) return -1;
+        s->test_ad_slots = slots > 0 ? std::max(64, slots / 64 * 64) : 0;
+        s->test_ad_tail = tail;
+        s->test_ad_alloc = alloc_slots > 0 ? alloc_slots : INT_MAX;
         return 0;
     });
 }

@@ -86,6 +86,7 @@ constexpr int AD_STAGE_BLOCK = 256;
 #ifndef AD_BOUNCE_WAVES
 #define AD_BOUNCE_WAVES (kF64 ? 1 : 2)
 #endif
+#define AD_TAIL_WAVES 1   // it runs too few paths to fill the chip
 #ifndef AD_EDGE_WAVES
 #define AD_EDGE_WAVES (kF64 ? 1 : 2)
 #endif
@@ -1418,6 +1419,22 @@ template <class K> static unsigned residentBlocks(K fn, unsigned blk, size_t lds
     }
     return (unsigned)std::max(ncu, 1) * (unsigned)per;
 }
+// A staged AD kernel's launch: its dynamic LDS with the part of the tree in it, and its grid.
+struct StageLaunch {
+    RenderParams P;
+    size_t lds = 0;
+    unsigned resident = 0;
+    template <class K> void set(K kern, const DScene &S, const RenderParams &P_, bool prefix) {
+        P = P_;
+        lds = traceLds(AD_STAGE_BLOCK, S.stack_depth);
+        lds += treeLdsFor(kern, AD_STAGE_BLOCK, S, P, prefix);
+        resident = residentBlocks(kern, AD_STAGE_BLOCK, lds);
+    }
+    unsigned blocks(uint32_t items) const {   // those beyond get no item (ListShare)
+        const unsigned least = 4 * (AD_STAGE_BLOCK / 64);
+        return std::min(resident, (items + least - 1) / least);
+    }
+};
 // The lists and counters of the staged AD kernels behind the path state (adStateBytes).
 struct AdLists {
     uint32_t *alive[2], *edges, *cnt;
@@ -1429,36 +1446,56 @@ struct AdLists {
         cnt = l + 3 * (size_t)P.ad_slots;
     }
 };
+// Whether no path is left before bounce k. Asked every 16 bounces, where as many launches or
+// more could follow (an empty one costs 2 to 5 us, the answer about 20): of a host that may
+// wait (P.ad_ask), not under capture.
+static bool allEnded(const RenderParams &P, const AdLists &ls, int k, hipStream_t sm) {
+    if (!P.ad_ask || k == 0 || k % 16 != 0 || P.max_bounces - k < 16) return false;
+    uint32_t left = 1;
+    return hipMemcpyAsync(&left, ls.cnt + 4 * k * AD_CNT, 4, hipMemcpyDeviceToHost, sm) == hipSuccess &&
+           hipStreamSynchronize(sm) == hipSuccess && left == 0;
+}
 // A VolPathTracerAD chunk as batches of at most P.ad_slots samples: per bounce one launch
 // of k_ad_bounce and one of k_ad_edges over the paths that are still alive.
 template <int N> void WidthOps<N>::launchAdStages(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n,
                                                   const uint4 *replay, real *acc, char *q, unsigned *qc, unsigned *st,
                                                   uint4 *ovf, unsigned *ovf_count, unsigned long long *wk, hipStream_t sm) {
-    const unsigned blk = AD_STAGE_BLOCK, wpb = blk / 64;
-    RenderParams Pb = P, Pe = P;
-    const size_t lb = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_bounce<N>, blk, S, Pb, treePrefixInLds<N>());
-    const size_t le = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_edges<N>, blk, S, Pe, treePrefixInLds<N>());
-    const unsigned rb = residentBlocks(k_ad_bounce<N>, blk, lb), re = residentBlocks(k_ad_edges<N>, blk, le);
+    const unsigned blk = AD_STAGE_BLOCK;
     const bool edges = P.sppse > 0 && S.edges_valid && (P.mode & (4 | 32)) != 0;
+    // launches of the kernels that this chunk needs (their occupancy queries cost about 25 us each)
+    StageLaunch bounce, edge, tail;
+    if (std::min<uint64_t>(n, P.ad_slots) > P.ad_tail) {
+        bounce.set(k_ad_bounce<N>, S, P, treePrefixInLds<N>());
+        if (edges) edge.set(k_ad_edges<N>, S, P, treePrefixInLds<N>());
+    }
+    if (P.ad_tail > 0) tail.set(k_ad_tail<N, AdPass::FORWARD, true>, S, P, treePrefixInLds<N>());
     const AdLists ls(P, AdSlots<N>::BYTES);
     AdBatch B{};
     B.state = P.ad_state;
     B.n = P.ad_slots;
     B.edges = ls.edges;
+    B.tail = P.ad_tail;
     for (uint64_t b0 = 0; b0 < n; b0 += B.n) {
         B.m = (uint32_t)std::min<uint64_t>(B.n, n - b0);
         B.s0 = s0 + b0;
         B.replay = replay ? replay + b0 : nullptr;
         (void)launch_fill32(ls.cnt, 4 * (P.max_bounces + 3) * AD_CNT, 0u, sm);
-        const unsigned few = (B.m + 4 * wpb - 1) / (4 * wpb);   // blocks beyond get no item (ListShare)
-        for (int k = 0; k <= P.max_bounces; ++k) {
+        for (int k = 0; B.m > B.tail && k <= P.max_bounces && !allEnded(P, ls, k, sm); ++k) {
             B.start = k == 0;
             B.in = k == 0 ? nullptr : ls.alive[k & 1];
             B.out = ls.alive[(k + 1) & 1];
             B.cnt = ls.cnt + 4 * k * AD_CNT;
-            hipLaunchKernelGGL(k_ad_bounce<N>, dim3(std::min(rb, few)), dim3(blk), lb, sm, S, Pb, B, q, qc, st, wk);
+            hipLaunchKernelGGL(k_ad_bounce<N>, dim3(bounce.blocks(B.m)), dim3(blk), bounce.lds, sm, S, bounce.P, B, q, qc, st, wk);
             if (edges && k < P.max_bounces)
-                hipLaunchKernelGGL(k_ad_edges<N>, dim3(std::min(re, few)), dim3(blk), le, sm, S, Pe, B, q, qc, st, wk);
+                hipLaunchKernelGGL(k_ad_edges<N>, dim3(edge.blocks(B.m)), dim3(blk), edge.lds, sm, S, edge.P, B, q, qc, st, wk);
+        }
+        if (B.tail > 0) {
+            B.start = B.m <= B.tail;
+            B.in = ls.alive[0];
+            B.out = ls.alive[1];
+            B.cnt = ls.cnt;
+            hipLaunchKernelGGL((k_ad_tail<N, AdPass::FORWARD, true>), dim3(tail.blocks(std::min(B.m, B.tail))), dim3(blk), tail.lds, sm, S,
+                               tail.P, B, q, qc, nullptr, 0, st, wk);
         }
         hipLaunchKernelGGL(k_ad_finish<N>, dim3((B.m + 255) / 256, 3 * (N + 1)), dim3(256), 0, sm, P, B, acc, ovf, ovf_count);
     }
@@ -1511,6 +1548,7 @@ template <int N> hipError_t WidthOps<N>::kernelInfo(KernelInfo *out, int cap, in
     }
     DT_INFO(k_ad_bounce<N>, "k_ad_bounce", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
     DT_INFO(k_ad_edges<N>, "k_ad_edges", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
+    DT_INFO((k_ad_tail<N, AdPass::FORWARD, true>), "k_ad_tail", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK))
     DT_INFO(k_ad_finish<N>, "k_ad_finish", 256, 0)
     DT_INFO((k_ad_paths<N, AD_PATH>), "k_ad_paths/path", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_ad_paths<N, AD_DIRECT>), "k_ad_paths/direct", MAX_BLOCK, traceLds(MAX_BLOCK))
@@ -1535,40 +1573,61 @@ void AdjointOps::launch(const DScene &S_, const RenderParams &P, uint64_t s0, ui
     constexpr int N = 1;
     DScene S = S_;
     S.nder = N;
-    const unsigned blk = AD_STAGE_BLOCK, wpb = blk / 64;
-    RenderParams Pb = P, Pa = P;
-    const size_t lb = traceLds(blk, S.stack_depth) + treeLdsFor(k_ad_bounce<N>, blk, S, Pb, treePrefixInLds<N>());
-    const size_t la = traceLds(blk, S.stack_depth) + treeLdsFor(k_adj_bounce<N>, blk, S, Pa, treePrefixInLds<N>());
-    const unsigned rb = residentBlocks(k_ad_bounce<N>, blk, lb), ra = residentBlocks(k_adj_bounce<N>, blk, la);
+    const unsigned blk = AD_STAGE_BLOCK;
+    StageLaunch bounce[2], tail[2];   // of each pass
+    if (std::min<uint64_t>(n, P.ad_slots) > P.ad_tail) {
+        bounce[0].set(k_ad_bounce<N>, S, P, treePrefixInLds<N>());
+        bounce[1].set(k_adj_bounce<N>, S, P, treePrefixInLds<N>());
+    }
+    if (P.ad_tail > 0) {
+        tail[0].set(k_ad_tail<N, AdPass::FORWARD, false>, S, P, treePrefixInLds<N>());
+        tail[1].set(k_ad_tail<N, AdPass::SCATTER, false>, S, P, treePrefixInLds<N>());
+    }
     const AdLists ls(P, AdSlots<N>::BYTES);
     AdBatch B{};
     B.state = P.ad_state;
     B.n = P.ad_slots;
+    B.tail = P.ad_tail;
     for (uint64_t b0 = 0; b0 < n; b0 += B.n) {
         B.m = (uint32_t)std::min<uint64_t>(B.n, n - b0);
         B.s0 = s0 + b0;
-        const unsigned few = (B.m + 4 * wpb - 1) / (4 * wpb);
+        const uint32_t mt = std::min(B.m, B.tail);
         for (int pass = 0; pass < 2; ++pass) {
             (void)launch_fill32(ls.cnt, 4 * (P.max_bounces + 3) * AD_CNT, 0u, sm);
             B.out = ls.alive[0];
             B.cnt = ls.cnt;
             hipLaunchKernelGGL(k_adj_list<N>, dim3((B.m + 255) / 256), dim3(256), 0, sm, S, B, dimg, pass);
-            for (int k = 0; k <= P.max_bounces; ++k) {
+            for (int k = 0; B.m > B.tail && k <= P.max_bounces && !allEnded(P, ls, k, sm); ++k) {
                 B.start = k == 0;
                 B.in = ls.alive[k & 1];
                 B.out = ls.alive[(k + 1) & 1];
                 B.cnt = ls.cnt + 4 * k * AD_CNT;
                 if (pass == 0)
-                    hipLaunchKernelGGL(k_ad_bounce<N>, dim3(std::min(rb, few)), dim3(blk), lb, sm, S, Pb, B, nullptr, nullptr, st, wk);
+                    hipLaunchKernelGGL(k_ad_bounce<N>, dim3(bounce[0].blocks(B.m)), dim3(blk), bounce[0].lds, sm, S, bounce[0].P, B, nullptr,
+                                       nullptr, st, wk);
                 else
-                    hipLaunchKernelGGL(k_adj_bounce<N>, dim3(std::min(ra, few)), dim3(blk), la, sm, S, Pa, B, grad, pmed, st, wk);
+                    hipLaunchKernelGGL(k_adj_bounce<N>, dim3(bounce[1].blocks(B.m)), dim3(blk), bounce[1].lds, sm, S, bounce[1].P, B, grad, pmed,
+                                       st, wk);
             }
+            if (B.tail == 0) continue;
+            B.start = 0;
+            B.in = ls.alive[0];
+            B.out = ls.alive[1];
+            B.cnt = ls.cnt;
+            if (pass == 0)
+                hipLaunchKernelGGL((k_ad_tail<N, AdPass::FORWARD, false>), dim3(tail[0].blocks(mt)), dim3(blk), tail[0].lds, sm, S, tail[0].P, B,
+                                   nullptr, nullptr, nullptr, 0, st, wk);
+            else
+                hipLaunchKernelGGL((k_ad_tail<N, AdPass::SCATTER, false>), dim3(tail[1].blocks(mt)), dim3(blk), tail[1].lds, sm, S, tail[1].P, B,
+                                   nullptr, nullptr, grad, pmed, st, wk);
         }
     }
 }
 hipError_t AdjointOps::kernelInfo(KernelInfo *out, int cap, int *count) {
     hipError_t e = addKernelInfo(k_ad_bounce<1>, "k_ad_bounce<1>/adjoint", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_ad_tail<1, AdPass::FORWARD, false>, "k_ad_tail<1>/adjoint", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_adj_bounce<1>, "k_adj_bounce<1>", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK), out, cap, count);
+    if (e == hipSuccess) e = addKernelInfo(k_ad_tail<1, AdPass::SCATTER, false>, "k_adj_tail<1>", AD_STAGE_BLOCK, traceLds(AD_STAGE_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_adj_list<1>, "k_adj_list<1>", 256, 0, out, cap, count);
     return e;
 }

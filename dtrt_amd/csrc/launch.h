@@ -22,6 +22,8 @@ struct RenderParams {
     int lds_nodes, lds_tris;     // set per launch: the part of the BVH the kernel copies into LDS (treeToLds)
     char *ad_state;              // path state of the staged AD kernels (adStateBytes) and the samples it holds at once
     unsigned ad_slots;
+    unsigned ad_tail;            // lists of at most so many paths run to their ends in one launch (k_ad_tail)
+    int ad_ask;                  // the host may wait for the lists' lengths
     int tree_in_hbm;             // nonzero: no part of the BVH goes into LDS (a test setting)
 };
 

@@ -88,6 +88,7 @@ _lib.dtrt_test_kernel_times.argtypes = [_P, C.POINTER(C.c_double), C.POINTER(C.c
 _lib.dtrt_test_scene_info.argtypes = [_P, C.POINTER(C.c_int64)]
 _lib.dtrt_test_set_queue_budget.argtypes = [_P, C.c_uint64]
 _lib.dtrt_test_set_tree_in_hbm.argtypes = [_P, C.c_int]
+_lib.dtrt_test_set_ad_batch.argtypes = [_P, C.c_int, C.c_int, C.c_int]
 _lib.dtrt_test_set_voxel_lanes.argtypes = [_P, C.c_int, C.POINTER(C.c_int), C.c_int]
 _lib.dtrt_scene_set_density.argtypes = [_P, C.c_int, _P, C.c_int]
 _lib.dtrt_scene_capture_views.argtypes = [_P, C.c_int, C.POINTER(_P), C.POINTER(_m.fns["render"].argtypes[2]._type_),
@@ -329,6 +330,12 @@ def set_voxel_lanes(scene, medium, voxels):
 def set_queue_budget(scene, nbytes):
     """Child-record queue bytes for this scene's renders (0 restores the default)."""
     _chk(_lib.dtrt_test_set_queue_budget(scene._h, int(nbytes)), "set_queue_budget")
+
+
+def set_ad_batch(scene, slots=0, tail=-1, alloc_slots=0):
+    """Samples in flight at once (0: default), the longest list that runs to its paths' ends in
+    one launch (-1: default), and the most samples whose path state can be allocated (0: any)."""
+    _chk(_lib.dtrt_test_set_ad_batch(scene._h, int(slots), int(tail), int(alloc_slots)), "set_ad_batch")
 
 
 def set_tree_in_hbm(scene, on=True):

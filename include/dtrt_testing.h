@@ -35,6 +35,12 @@ int dtrt_test_set_queue_budget(dtrt_object *scene, uint64_t bytes);
  * keeps the tree, or its top levels, in LDS where that costs no occupancy. Images are
  * the same either way up to summation order. */
 int dtrt_test_set_tree_in_hbm(dtrt_object *scene, int on);
+/* How VolPathTracerAD and the density adjoint run the scene's samples (0, -1, 0: the
+ * defaults). slots > 0: at most so many samples (in whole 64s, at least 64) in flight at once, so
+ * that a chunk runs as several batches; tail >= 0: lists of at most so many paths run to their
+ * ends in one launch (0: none do, every bounce is a launch of its own); alloc_slots > 0: path
+ * state for more samples cannot be allocated. Results are the same up to summation order. */
+int dtrt_test_set_ad_batch(dtrt_object *scene, int slots, int tail, int alloc_slots);
 /* [0] BVH nodes, [1] triangles, [2] edges, [3] primary edges, [4] primary-edge
  * length sum (double bits), [5] secondary edges usable, [6] vertices, [7] faces. */
 int dtrt_test_scene_info(dtrt_object *scene, int64_t *out8);
