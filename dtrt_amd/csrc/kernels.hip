@@ -72,6 +72,15 @@ HDI unsigned blockOr64(int b) { return b == 128 || b == 256 ? (unsigned)b : 64u;
 // price of spills. 100K-face dielectric scene, child kernel at 8 lanes 36.7 ms with 2 waves per
 // SIMD, 41.5 with 3, 32.8 with 4, 39.1 with 5; surface scene's tree read from HBM 70.5 -> 62.7 ms.
 #define CHILD_WAVES_HBM 4
+// The spills cost where few paths run to great depth, or too few to fill four waves per SIMD:
+// there the kernels have the other trees' waves (FEW). Children of the 25K-face dielectric scene in
+// double with 2 against 4 waves: 313K records at limits of 24, 50 and 200 bounces 7.3 against 8.7 ms, 12.0
+// against 14.2, 23.1 against 25.9 (a wave per SIMD more costs every step of the longest path); 1.8M records
+// at 6 bounces 14.7 against 13.9, at 50 31.0 against 32.7; of 100K faces, 2.7M at 16 and 32 bounces 40.6
+// against 36.6 and 52.6 against 48.0. They cross at 30K (100K faces) to 80K records per bounce of the limit.
+constexpr bool kFew = CHILD_WAVES_PER_SIMD != CHILD_WAVES_HBM;
+constexpr unsigned CHILD_FEW_PER_BOUNCE = 50000;
+constexpr int childWaves(bool hbm, bool few) { return hbm && !few ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD; }
 #ifndef AD_WAVES_PER_SIMD
 #define AD_WAVES_PER_SIMD (kF64 ? 1 : 2)   // the surface-only AD kernel
 #endif
@@ -569,8 +578,8 @@ __global__ __launch_bounds__(MAX_BLOCK, adWaves<N>()) void k_ad_paths(DScene S, 
 //   PRIMAL_PATH     PathTracer (path.cpp:64-96) and DirectIntegrator (direct.cpp:
 //                   51-85, max depth 1): pathStep, camera ray from tnear ShadowEpsilon.
 // Radiance sums go to acc[pixel][3].
-template <int KIND, Tree WHERE>
-__global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD) void k_primal_paths(DScene S, RenderParams P, uint64_t s0,
+template <int KIND, Tree WHERE, bool FEW = false>
+__global__ __launch_bounds__(WIDE_BLOCK, childWaves(WHERE == Tree::HBM, FEW)) void k_primal_paths(DScene S, RenderParams P, uint64_t s0,
                                                                                      uint64_t nsamp, real *acc,
                                                                                      unsigned long long *work) {
     const uint32_t blk = xcdRemap(blockIdx.x, gridDim.x);
@@ -947,11 +956,12 @@ DI int lanesToUse(unsigned n) {
 // Persistent: each lane holds one primal sub-path and advances it one bounce per
 // iteration; a lane whose path has ended takes the next queued record (one atomic
 // per wave on qnext), so the lanes of a wave stay busy until the queue is drained.
-template <int N, Tree WHERE>
-__global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
+template <int N, Tree WHERE, bool FEW = false>
+__global__ __launch_bounds__(WIDE_BLOCK, childWaves(WHERE == Tree::HBM, FEW)) void k_children(DScene S, RenderParams P, const char *q, const unsigned *qcount,
                                                     unsigned *qnext, real *acc, real *acc_pe, unsigned long long *work) {
     const unsigned n = min(*qcount, P.qcap);
     if (blockIdx.x >= n) return;   // each block before this one has a record
+    if (WHERE == Tree::HBM && (FEW ? n > P.child_few : n <= P.child_few)) return;   // the other one's queue
     Tracer<N, WHERE> T(S);
     T.useLdsTree(P);
     const int lane = threadIdx.x & 63;
@@ -1014,13 +1024,14 @@ __global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : 
 
 // Persistent drain of CHILD_PATH records (the surface-only integrators' sub-paths,
 // path.cpp:11-61 from the record's origin and direction), as k_children.
-template <int N, Tree WHERE>
-__global__ __launch_bounds__(WIDE_BLOCK, WHERE == Tree::HBM ? CHILD_WAVES_HBM : CHILD_WAVES_PER_SIMD) void k_children_path(DScene S, RenderParams P, const char *q,
+template <int N, Tree WHERE, bool FEW = false>
+__global__ __launch_bounds__(WIDE_BLOCK, childWaves(WHERE == Tree::HBM, FEW)) void k_children_path(DScene S, RenderParams P, const char *q,
                                                                             const unsigned *qcount, unsigned *qnext,
                                                                             real *acc, real *acc_pe,
                                                                             unsigned long long *work) {
     const unsigned n = min(*qcount, P.qcap);
     if (blockIdx.x >= n) return;   // each block before this one has a record
+    if (WHERE == Tree::HBM && (FEW ? n > P.child_few : n <= P.child_few)) return;   // the other one's queue
     Tracer<N, WHERE> T(S);
     T.useLdsTree(P);
     const int lane = threadIdx.x & 63;
@@ -1370,6 +1381,17 @@ template <class K> static size_t treeLdsFor(K kern, unsigned blk, const DScene &
     return tb;
 }
 
+// Blocks of `blk` threads and `lds` bytes of kernel `fn` that the device holds at once.
+template <class K> static unsigned residentBlocks(K fn, unsigned blk, size_t lds) {
+    int dev = 0, ncu = 0, per = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, (int)blk, lds) != hipSuccess || per <= 0) {
+        (void)hipGetLastError();
+        per = 1;
+    }
+    return (unsigned)std::max(ncu, 1) * (unsigned)per;
+}
 // The work-group size of a launch of `kern` whose default is `blk`: WIDE_BLOCK where only that
 // many waves, sharing one copy, leave room for the whole tree.
 template <class K> static unsigned wideGroup(K kern, unsigned blk, const DScene &S, const RenderParams &P) {
@@ -1407,17 +1429,6 @@ template <int N> void WidthOps<N>::launchAd(const DScene &S, const RenderParams 
     } else {
         launchAdStages(S, P, s0, n, replay, acc, q, qc, st, ovf, ovf_count, wk, sm);
     }
-}
-// Blocks of `blk` threads and `lds` bytes of kernel `fn` that the device holds at once.
-template <class K> static unsigned residentBlocks(K fn, unsigned blk, size_t lds) {
-    int dev = 0, ncu = 0, per = 0;
-    (void)hipGetDevice(&dev);
-    (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, (int)blk, lds) != hipSuccess || per <= 0) {
-        (void)hipGetLastError();
-        per = 1;
-    }
-    return (unsigned)std::max(ncu, 1) * (unsigned)per;
 }
 // A staged AD kernel's launch: its dynamic LDS with the part of the tree in it, and its grid.
 struct StageLaunch {
@@ -1506,21 +1517,22 @@ template <int N> void WidthOps<N>::launchChildren(const DScene &S, const RenderP
     // launched, since each drains the queue until it is empty
     const unsigned dflt = blockOr64(P.child_block);
     RenderParams Pl = P;
-    auto launch = [&](auto in_lds, auto in_hbm) {
-        unsigned blk = wideGroup(in_lds, dflt, S, P);
-        size_t tree = treeLdsFor(in_lds, blk, S, Pl, false);
-        auto kern = in_lds;
-        if (!Pl.lds_tris) {
-            kern = in_hbm;
-            blk = dflt;
-            tree = treeLdsFor(in_hbm, blk, S, Pl, true);
-        }
+    auto drain = [&](auto kern, unsigned blk, size_t tree) {
         const size_t lds = traceLds(blk, S.stack_depth) + tree;
         const unsigned nb = std::min(std::max(1u, grid * dflt / blk), residentBlocks(kern, blk, lds));
         hipLaunchKernelGGL(kern, dim3(nb), dim3(blk), lds, sm, S, Pl, q, qc, qc + 2, acc, acc_pe, wk);
     };
-    if (P.ad_kind == AD_VOLPATH) launch(k_children<N, Tree::LDS>, k_children<N, Tree::HBM>);
-    else launch(k_children_path<N, Tree::LDS>, k_children_path<N, Tree::HBM>);
+    auto launch = [&](auto in_lds, auto in_hbm, auto in_hbm_few) {
+        const unsigned blk = wideGroup(in_lds, dflt, S, P);
+        const size_t tree = treeLdsFor(in_lds, blk, S, Pl, false);
+        if (Pl.lds_tris) return drain(in_lds, blk, tree);
+        // the queue's length is on the device: one of the two takes it, the other one's blocks leave
+        Pl.child_few = kFew ? CHILD_FEW_PER_BOUNCE * (unsigned)P.max_bounces : 0;
+        drain(in_hbm, dflt, treeLdsFor(in_hbm, dflt, S, Pl, true));
+        if (kFew) drain(in_hbm_few, dflt, treeLdsFor(in_hbm_few, dflt, S, Pl, true));
+    };
+    if (P.ad_kind == AD_VOLPATH) launch(k_children<N, Tree::LDS>, k_children<N, Tree::HBM>, k_children<N, Tree::HBM, kFew>);
+    else launch(k_children_path<N, Tree::LDS>, k_children_path<N, Tree::HBM>, k_children_path<N, Tree::HBM, kFew>);
 }
 template <int N> void WidthOps<N>::launchPrimary(const DScene &S, const RenderParams &P, int view, uint64_t s0, uint64_t n,
                                            uint64_t total, char *q, unsigned *qc, unsigned *st, unsigned long long *wk,
@@ -1554,8 +1566,10 @@ template <int N> hipError_t WidthOps<N>::kernelInfo(KernelInfo *out, int cap, in
     DT_INFO((k_ad_paths<N, AD_DIRECT>), "k_ad_paths/direct", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_children<N, Tree::LDS>), "k_children", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_children<N, Tree::HBM>), "k_children/hbm", MAX_BLOCK, traceLds(MAX_BLOCK))
+    if (kFew) DT_INFO((k_children<N, Tree::HBM, kFew>), "k_children/hbm/few", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_children_path<N, Tree::LDS>), "k_children_path", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO((k_children_path<N, Tree::HBM>), "k_children_path/hbm", MAX_BLOCK, traceLds(MAX_BLOCK))
+    if (kFew) DT_INFO((k_children_path<N, Tree::HBM, kFew>), "k_children_path/hbm/few", MAX_BLOCK, traceLds(MAX_BLOCK))
     DT_INFO(k_primary<N>, "k_primary", PRIMARY_BLOCK, traceLds(PRIMARY_BLOCK))
     DT_INFO(k_grid<N>, "k_grid", BLOCK, 0)
     DT_INFO(k_finalize<N>, "k_finalize", 256, 0)
@@ -1734,22 +1748,31 @@ hipError_t launch_primal_paths(const DScene &S, const RenderParams &P, int kind,
     if ((n + PRIMAL_BLOCK - 1) / PRIMAL_BLOCK > 0x7FFFFFFFull) return hipErrorInvalidValue;
     real *A = static_cast<real *>(acc);
     RenderParams Pl = P;
-    auto launch = [&](auto in_lds, auto in_hbm) {
+    auto launch = [&](auto in_lds, auto in_hbm, auto in_hbm_few) {
         unsigned blk = wideGroup(in_lds, PRIMAL_BLOCK, S, P);
         size_t tree = treeLdsFor(in_lds, blk, S, Pl, false);
         auto kern = in_lds;
         if (!Pl.lds_tris) {
-            kern = in_hbm;
+            // samples that two waves per SIMD hold at once get no more waves by a third: 50K-face scene,
+            // 10 bounces, VolPathTracer of 129,600 samples 1.65 ms with 2 waves, 2.08 with 4; of 147,456 2.47 and 2.29
             blk = PRIMAL_BLOCK;
-            tree = treeLdsFor(in_hbm, blk, S, Pl, true);
+            kern = in_hbm_few;
+            tree = treeLdsFor(kern, blk, S, Pl, true);
+            if (kFew && n > (uint64_t)blk * residentBlocks(kern, blk, traceLds(blk, S.stack_depth) + tree)) {
+                kern = in_hbm;
+                tree = treeLdsFor(kern, blk, S, Pl, true);
+            }
         }
         hipLaunchKernelGGL(kern, dim3((unsigned)((n + blk - 1) / blk)), dim3(blk), traceLds(blk, S.stack_depth) + tree, sm, S, Pl, s0, n,
                            A, work);
         return hipGetLastError();
     };
-    if (kind == PRIMAL_SIMPLE) return launch(k_primal_paths<PRIMAL_SIMPLE, Tree::LDS>, k_primal_paths<PRIMAL_SIMPLE, Tree::HBM>);
-    if (kind == PRIMAL_PATH) return launch(k_primal_paths<PRIMAL_PATH, Tree::LDS>, k_primal_paths<PRIMAL_PATH, Tree::HBM>);
-    if (kind == PRIMAL_VOLPATH) return launch(k_primal_paths<PRIMAL_VOLPATH, Tree::LDS>, k_primal_paths<PRIMAL_VOLPATH, Tree::HBM>);
+    if (kind == PRIMAL_SIMPLE)
+        return launch(k_primal_paths<PRIMAL_SIMPLE, Tree::LDS>, k_primal_paths<PRIMAL_SIMPLE, Tree::HBM>, k_primal_paths<PRIMAL_SIMPLE, Tree::HBM, kFew>);
+    if (kind == PRIMAL_PATH)
+        return launch(k_primal_paths<PRIMAL_PATH, Tree::LDS>, k_primal_paths<PRIMAL_PATH, Tree::HBM>, k_primal_paths<PRIMAL_PATH, Tree::HBM, kFew>);
+    if (kind == PRIMAL_VOLPATH)
+        return launch(k_primal_paths<PRIMAL_VOLPATH, Tree::LDS>, k_primal_paths<PRIMAL_VOLPATH, Tree::HBM>, k_primal_paths<PRIMAL_VOLPATH, Tree::HBM, kFew>);
     return hipErrorInvalidValue;
 }
 hipError_t launch_particles(const DScene &S, const RenderParams &P, uint64_t s0, uint64_t n, void *acc,
@@ -1795,10 +1818,13 @@ hipError_t kernel_info(const DScene &S, KernelInfo *out, int cap, int *count) {
     if (e == hipSuccess) e = AdjointOps::kernelInfo(out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::LDS>, "k_primal_paths/volpath", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::HBM>, "k_primal_paths/volpath/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (kFew && e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_VOLPATH, Tree::HBM, kFew>, "k_primal_paths/volpath/hbm/few", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE, Tree::LDS>, "k_primal_paths/simple", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE, Tree::HBM>, "k_primal_paths/simple/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (kFew && e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_SIMPLE, Tree::HBM, kFew>, "k_primal_paths/simple/hbm/few", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_PATH, Tree::LDS>, "k_primal_paths/path", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_PATH, Tree::HBM>, "k_primal_paths/path/hbm", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
+    if (kFew && e == hipSuccess) e = addKernelInfo(k_primal_paths<PRIMAL_PATH, Tree::HBM, kFew>, "k_primal_paths/path/hbm/few", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_particles, "k_particles", PRIMAL_BLOCK, traceLds(PRIMAL_BLOCK), out, cap, count);
     if (e == hipSuccess) e = addKernelInfo(k_refit, "k_refit", 256, 0, out, cap, count);
     return e;

@@ -20,6 +20,7 @@ struct RenderParams {
     unsigned qcap;           // child records the queue can hold
     int ad_block, child_block;   // work-group sizes of the AD-path and child kernels (64, 128, 256; 0 = 64)
     int lds_nodes, lds_tris;     // set per launch: the part of the BVH the kernel copies into LDS (treeToLds)
+    unsigned child_few;          // set per launch: the longest queue of the child kernels with FEW
     char *ad_state;              // path state of the staged AD kernels (adStateBytes) and the samples it holds at once
     unsigned ad_slots;
     unsigned ad_tail;            // lists of at most so many paths run to their ends in one launch (k_ad_tail)
