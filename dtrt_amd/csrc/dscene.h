@@ -118,25 +118,38 @@ DI void treeToLds(const DScene &S, int lds_nodes, bool lds_tris) {
     __syncthreads();
 }
 
-// The two children's entry distances (at least tnear) and whether the ray (origin o,
-// reciprocal direction inv) meets their boxes in [tnear, tfar]. n*: the planes it enters
-// by, f*: those it leaves by, each {left, right}. Choosing them by the direction's sign
-// replaces a minimum and a maximum per plane pair; the distances are the same, but for a ray
-// with a zero direction component whose origin lies in a box plane: there one plane's
-// distance is 0 * inf. in_plane (wave-uniform: some lane's ray has such a component) orders
-// the pairs all the same, and the ray is outside unless the box is flat: about one float
-// camera ray in 65,536 of an odd-sized image's middle column lies in such a plane.
-struct Hit2 { bool l, r; };
+// Where a ray (origin o, reciprocal direction inv) has a zero direction component, a box plane
+// that holds its origin is at the distance 0 * inf. A slab test by minimum and maximum per plane pair
+// then puts the ray outside, unless the box is flat (about one float camera ray in 65,536 of an
+// odd-sized image's middle column lies in such a plane). Planes chosen by sign keep that answer in
+// one of two ways. In kernels with the tree in LDS, whose registers are full, some lane's infinite
+// inv has the wave order the pairs all the same (in_plane): cube render's children 190 ms, 197 with the
+// other way. In the others, which wait for their nodes, the origin is the next number before it for
+// the planes the ray enters by, and the next one behind it for those it leaves by: children at 2.8M
+// records and 24 bounces 34.2 ms, 34.7 with the first way; VolPathTracer of 524K samples at 200 bounces
+// 21.6 and 22.4. (A flat box that holds the ray is then missed, but so are its triangles, which are
+// parallel to the ray.)
+DI float besideOrigin(float o, float inv, bool before) {
+    if (!isinf(inv)) return o;
+    const bool up = (inv < 0.f) == before;
+    if (o == 0.f) return up ? __FLT_DENORM_MIN__ : -__FLT_DENORM_MIN__;
+    return __int_as_float(__float_as_int(o) + ((o > 0.f) == up ? 1 : -1));
+}
 DI void orderPlanes(float2 &n, float2 &f) {
     const float2 a = n, b = f;
     n = float2{fminf(a.x, b.x), fminf(a.y, b.y)};
     f = float2{fmaxf(a.x, b.x), fmaxf(a.y, b.y)};
 }
-DI Hit2 boxesHit(fv3 o, fv3 inv, float2 nx, float2 ny, float2 nz, float2 fx, float2 fy, float2 fz, float tnear, float tfar,
+// The two children's entry distances (at least tnear) and whether the ray meets their boxes in
+// [tnear, tfar]. n*: the planes it enters by, from origin on, f*: those it leaves by, from of, each
+// {left, right}. Choosing them by the direction's sign replaces a minimum and a maximum per plane
+// pair; the distances are the same.
+struct Hit2 { bool l, r; };
+DI Hit2 boxesHit(fv3 on, fv3 of, fv3 inv, float2 nx, float2 ny, float2 nz, float2 fx, float2 fy, float2 fz, float tnear, float tfar,
                  bool in_plane, float &tl, float &tr) {
-    nx = float2{(nx.x - o.x) * inv.x, (nx.y - o.x) * inv.x}; fx = float2{(fx.x - o.x) * inv.x, (fx.y - o.x) * inv.x};
-    ny = float2{(ny.x - o.y) * inv.y, (ny.y - o.y) * inv.y}; fy = float2{(fy.x - o.y) * inv.y, (fy.y - o.y) * inv.y};
-    nz = float2{(nz.x - o.z) * inv.z, (nz.y - o.z) * inv.z}; fz = float2{(fz.x - o.z) * inv.z, (fz.y - o.z) * inv.z};
+    nx = float2{(nx.x - on.x) * inv.x, (nx.y - on.x) * inv.x}; fx = float2{(fx.x - of.x) * inv.x, (fx.y - of.x) * inv.x};
+    ny = float2{(ny.x - on.y) * inv.y, (ny.y - on.y) * inv.y}; fy = float2{(fy.x - of.y) * inv.y, (fy.y - of.y) * inv.y};
+    nz = float2{(nz.x - on.z) * inv.z, (nz.y - on.z) * inv.z}; fz = float2{(fz.x - of.z) * inv.z, (fz.y - of.z) * inv.z};
     if (in_plane) {
         orderPlanes(nx, fx);
         orderPlanes(ny, fy);
@@ -166,7 +179,14 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
     const float BEPS = 1e-6f;
     const fv3 inv{1.0f / d.x, 1.0f / d.y, 1.0f / d.z};
     const bool ngx = inv.x < 0.f, ngy = inv.y < 0.f, ngz = inv.z < 0.f;   // entered by the high planes
-    const bool in_plane = __any(isinf(inv.x) || isinf(inv.y) || isinf(inv.z));
+    fv3 on = o, of = o;
+    bool in_plane = false;
+    if constexpr (WHERE == Tree::LDS) {
+        in_plane = __any(isinf(inv.x) || isinf(inv.y) || isinf(inv.z));
+    } else {
+        on = {besideOrigin(o.x, inv.x, true), besideOrigin(o.y, inv.y, true), besideOrigin(o.z, inv.z, true)};
+        of = {besideOrigin(o.x, inv.x, false), besideOrigin(o.y, inv.y, false), besideOrigin(o.z, inv.z, false)};
+    }
     float best = tfar;
     const float *lds = ldsTree(stack_depth);
     const float *lx = lds + (ngx ? 2 : 0), *ly = lds + (ngy ? 6 : 4), *lz = lds + (ngz ? 10 : 8);
@@ -208,7 +228,7 @@ DI TraceHit traceClosest(const float4 *nodes, const float4 *tris, int nnodes, f3
             }
             float tl, tr;
             nbox += 2;
-            const Hit2 hit = boxesHit(o, inv, nx, ny, nz, fx, fy, fz, tnear, best, in_plane, tl, tr);
+            const Hit2 hit = boxesHit(on, of, inv, nx, ny, nz, fx, fy, fz, tnear, best, in_plane, tl, tr);
             const bool hl = hit.l, hr = hit.r;
             const bool right = hr && (!hl || tr < tl);   // the right child is the next node
             top[stride] = right ? cl : cr;   // the other one; above the top unless both are hit
