@@ -663,8 +663,9 @@ struct Bump {
         return r;
     }
 };
-// The scratch-only render's child queue must hold at least this much; below it the
-// render is refused (the exact overflow replay would still finish, in many rounds).
+// The scratch-only render's child queue and VolPathTracerAD's path state, at most a quarter of
+// this, must hold at least this much together; below it the render is refused (the exact
+// overflow replay would still finish, in many rounds).
 constexpr uint64_t NOALLOC_MIN_QUEUE = uint64_t(16) << 20;
 // AD samples in flight at once (the slots of the staged AD kernels' path state).
 #ifndef AD_SLOTS_LOG
@@ -1483,11 +1484,13 @@ bool Scene::renderViews(int nv, const Camera *const *cams, const dtrt_render_opt
         if (!A || !APE || !qc || !st || !wk || !OV[0] || !OV[1] || qbytes < NOALLOC_MIN_QUEUE)
             return fail("render_device_noalloc: the image needs more than the " +
                         std::to_string(DTRT_SCRATCH_BYTES >> 20) + " MiB scratch area holds (accumulators " +
-                        std::to_string((img + (size_t)nder * npix * 3) * es >> 20) + " MiB, plus a queue of at least " +
+                        std::to_string((img + (size_t)nder * npix * 3) * es >> 20) + " MiB, plus a queue and path state of at least " +
                         std::to_string(NOALLOC_MIN_QUEUE >> 20) + " MiB)");
-        // a quarter of it for the path state, as many samples in flight as fit
-        P.ad_slots = (unsigned)std::min<uint64_t>(adSlots(), (qbytes / 4 - adStateBytes(nder, S.f64 != 0, 0)) / adSlotBytes(nder, S.f64 != 0) / 64 * 64);
-        P.ad_state = static_cast<char *>(pool->take(adStateBytes(nder, S.f64 != 0, P.ad_slots)));
+        if (ad_kind == AD_VOLPATH) {   // path state for a chunk's samples, or for as many as a quarter of it holds
+            const uint64_t fit = (qbytes / 4 - adStateBytes(nder, S.f64 != 0, 0)) / adSlotBytes(nder, S.f64 != 0) / 64 * 64;
+            P.ad_slots = (unsigned)std::min<uint64_t>({adSlots(), fit, (max_chunk + 63) / 64 * 64});
+            P.ad_state = static_cast<char *>(pool->take(adStateBytes(nder, S.f64 != 0, P.ad_slots)));
+        }
         const uint64_t qleft = pool->left / 256 * 256;
         Q = static_cast<char *>(pool->take(qleft));
         cap = std::min<uint64_t>(qleft / P.rec_stride, 0xFFFFFFF0ull);
