@@ -757,7 +757,8 @@ struct Scene : Obj {
     int tune_child_blocks = 32;
     double tune_fill = 0.75;
     uint64_t tune_max_chunk = uint64_t(1) << 22;
-    // work-group sizes of the AD-path and child kernels. The child kernel's 256 lets a
+    // work-group sizes of the AD-path kernels of the surface-only integrators and of the child
+    // kernels. The child kernel's 256 lets a
     // small scene's tree sit in LDS beside the traversal stacks at the kernel's full
     // occupancy (treeLdsFor in kernels.hip): benchmark scene 390 -> 318 ms in double,
     // 262 -> 220 ms in float, against 64.
@@ -2175,8 +2176,9 @@ bool Scene::autotune(const dtrt_render_options &o, int ad_kind, double *best_ms,
     };
     for (size_t q : budgets)
         if (!tryKnob(queue_budget, q)) return false;
-    for (int g : groups)
-        if (!tryKnob(tune_ad_block, g)) return false;
+    if (ad_kind != AD_VOLPATH)   // whose kernels have one size
+        for (int g : groups)
+            if (!tryKnob(tune_ad_block, g)) return false;
     for (int g : groups)
         if (!tryKnob(tune_child_block, g)) return false;
     for (int b : blocks) {

@@ -150,7 +150,8 @@ int dtrt_render_device(int integrator, dtrt_object *scene, const dtrt_render_opt
 
 /* Autotuner (no counterpart in the reference): renders `options` with the scene's
  * camera several times, by coordinate descent over the launch settings (child queue
- * budget, work-group sizes of the AD-path and child kernels, persistent child blocks
+ * budget, work-group sizes of the AD-path (PathTracerAD and DirectAD; VolPathTracerAD's
+ * have one size) and child kernels, persistent child blocks
  * per CU, the queue share an AD chunk aims at, the largest AD chunk), and
  * keeps the fastest in the scene for later renders, view batches and graph captures.
  * integrator: 0, 6 or 7. best_ms (may be NULL): the fastest render; settings3 (may be
