@@ -25,7 +25,7 @@ FLAGS = ["-O3", "-std=c++17", "-fPIC", "--offload-arch=" + ARCH, "-munsafe-fp-at
 
 # kernels.hip is compiled once per estimator precision (DT_REAL double in namespace
 # dt::p64, float in dt::p32) and, within each, once per dual width N (its AD, child,
-# primary-edge, adjoint and finalize kernels; each object holds its own
+# primary-edge and finalize kernels, with N = 1 the adjoint's; each object holds its own
 # frame-rotation constant) and once without DT_N (the width-independent kernels and
 # the dispatchers over nder). dispatch.cpp picks the precision, host.cpp is the C-ABI.
 WIDTHS = (16, 8, 4, 3, 2, 1)   # widest first: the longest compiles start first

@@ -297,7 +297,8 @@ int dtrt_scene_set_stream(dtrt_object *scene, void *stream);
  * [3] invalid edge weights, [4] non-orthogonal edge tangents, [5] medium
  * inconsistencies, [6] AD samples re-run after their child pushes overflowed the
  * queue (exact replay; the image is unaffected), [7] AD path samples,
- * [8] child sub-paths, [9] primary-edge samples. */
+ * [8] child sub-paths, [9] primary-edge samples. Edge samples on surfaces without
+ * reflectance, which can add nothing, are not drawn and not counted in [3] and [4]. */
 int dtrt_render_stats(dtrt_object *scene, int64_t *out10);
 
 #ifdef __cplusplus
