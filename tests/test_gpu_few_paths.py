@@ -43,3 +43,18 @@ def test_child_queues_of_either_length(gpu, integrator, nder, sppe):
     assert np.abs(lds[1]).max() > 0
     for lane in range(nder + 1):
         assert np.allclose(lds[lane], hbm[lane], rtol=1e-5, atol=1e-7 * np.abs(lds[lane]).max()), lane
+
+
+@pytest.mark.parametrize("nder,sppe", [(1, 200), (3, 60000)])
+def test_direct_child_queues_do_not_depend_on_the_limit(gpu, nder, sppe):
+    """DirectAD's children have one bounce: a limit of 50 gives the images of a limit of 2, in either kernel."""
+    d, sc = _surface(gpu, nder, 24, 4)
+    kw = dict(seed=3, scene=sc, sppe=sppe, integrator=gpu.DirectAD())
+    lds = scenes.render(gpu, d, max_bounces=2, **kw).astype(np.float64)
+    assert gpu.render_stats(sc)["children"] > 0
+    gpu.set_tree_in_hbm(sc, True)
+    assert np.abs(lds[1]).max() > 0
+    for limit in (2, 50):
+        hbm = scenes.render(gpu, d, max_bounces=limit, **kw).astype(np.float64)
+        for lane in range(nder + 1):
+            assert np.allclose(lds[lane], hbm[lane], rtol=1e-5, atol=1e-7 * np.abs(lds[lane]).max()), (limit, lane)
